@@ -246,6 +246,45 @@ __global__ __launch_bounds__(256) void rms_norm_row_kernel(const float * __restr
     }
 }
 
+// Narrow rows (d <= 256 floats, d % 4 == 0, 16-byte aligned, no packed
+// output): the per-head norms of q and k. A row is L lanes of one float4 each
+// (L the power of two that covers d), so a 256-thread workgroup holds 256/L
+// rows at once and ROWS of them a thread, every load issued before the first
+// sum. HBM bound: one workgroup per row, as the wider rows run, leaves 7 of 8
+// lanes idle at d = 128 and is bound by dispatching 65536 workgroups
+// (65536 x 128: 45.5 -> 11.6 us, 67 MB at 5.8 TB/s; 16384 x 128: 13.8 -> 5.9). The sums are
+// rms_norm_row_kernel's own: its lanes past the row add zeros.
+template <int L, int ROWS>
+__global__ __launch_bounds__(256) void rms_norm_narrow_kernel(const float * __restrict__ x, int64_t rows, int64_t d,
+                                                              float eps, const float * __restrict__ w,
+                                                              float * __restrict__ y) {
+    const int l = threadIdx.x % L, c = 4 * l;
+    const int64_t r0 = (int64_t) blockIdx.x * (256 / L * ROWS) + threadIdx.x / L;
+    const bool col = c < d;
+    float4 v[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const int64_t r = r0 + i * (256 / L);
+        v[i] = col && r < rows ? *reinterpret_cast<const float4 *>(x + r * d + c) : make_float4(0, 0, 0, 0);
+    }
+    const float4 wv = w && col ? *reinterpret_cast<const float4 *>(w + c) : make_float4(1, 1, 1, 1);
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const int64_t r = r0 + i * (256 / L);
+        float ss = 0.0f;
+        ss += v[i].x * v[i].x;
+        ss += v[i].y * v[i].y;
+        ss += v[i].z * v[i].z;
+        ss += v[i].w * v[i].w;
+#pragma unroll
+        for (int off = L / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+        const float sc = 1.0f / sqrtf(ss / (float) d + eps);
+        if (col && r < rows)
+            *reinterpret_cast<float4 *>(y + r * d + c) =
+                make_float4(v[i].x * sc * wv.x, v[i].y * sc * wv.y, v[i].z * sc * wv.z, v[i].w * sc * wv.w);
+    }
+}
+
 // One thread per 16 outputs of one row: y = act(g) * u (REGLU as g > 0 ? g*u : 0).
 // With a packed output the grid also covers its padding rows, written as zeros.
 template <int KIND>
@@ -396,6 +435,13 @@ dim3 row_grid(int64_t rows, int64_t d) {
 
 bool aligned16(const void * p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+template <int L>
+void rms_norm_narrow(const float * x, int64_t rows, int64_t d, float eps, const float * w, float * y, hipStream_t s) {
+    constexpr int ROWS = 4;
+    hipLaunchKernelGGL((rms_norm_narrow_kernel<L, ROWS>), dim3((unsigned) ((rows + 256 / L * ROWS - 1) / (256 / L * ROWS))),
+                       dim3(256), 0, s, x, rows, d, eps, w, y);
+}
+
 template <int OP>
 void binary_rows(const float * a, const float * b, int64_t rows, int64_t d, int b_row, float * y,
                         hipStream_t s) {
@@ -421,7 +467,12 @@ int zest_rms_norm(const float * x, int64_t rows, int64_t d, float eps, const flo
     const int64_t chunks = (zest_k_padded(d) + 255) / 256;  // the output pass covers the padded width
     hipStream_t s = zest::as_stream(stream);
     uint8_t * pk = (uint8_t *) packed;
-    if (chunks <= 4)  // up to 1024 columns: one workgroup per row
+    if (!packed && d <= 256 && d % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(w)) {
+        // several rows a workgroup
+        if (d > 128) rms_norm_narrow<64>(x, rows, d, eps, w, y, s);
+        else if (d > 64) rms_norm_narrow<32>(x, rows, d, eps, w, y, s);
+        else rms_norm_narrow<16>(x, rows, d, eps, w, y, s);
+    } else if (chunks <= 4)  // up to 1024 columns: one workgroup per row
         hipLaunchKernelGGL(rms_norm_row_kernel<1>, dim3((unsigned) grid_rows), dim3(256), 0, s, x, rows, d, eps, w, y,
                            pk, R_pad);
     else if (chunks <= 12)  // up to 3072

@@ -207,3 +207,28 @@ def test_expanded_writers_random_shapes(zest_gpu, oracle):
         assert _padding_is_zero(zest_gpu, host, rows, d), (rows, d)
     del torch
 
+
+
+@pytest.mark.parametrize("rows,d", [(1, 4), (3, 60), (65, 64), (257, 68), (33, 128), (1000, 128), (31, 132), (7, 252), (130, 256)])
+def test_rms_norm_narrow_rows(zest_gpu, oracle, rows, d):
+    """Rows of at most 256 floats, several a workgroup: against the oracle, and bit for bit what the
+    row-a-workgroup kernel gives (which rows that are not 16-byte aligned take); nothing past the rows is written."""
+    import torch
+    x = Rng(rows + d).normal(rows * d, 0, 1.5).reshape(rows, d)
+    w = Rng(d).normal(d, 1.0, 0.1)
+    x[0, :] = 0.0
+    if rows > 2:
+        x[2, d // 2] = np.inf
+    xt, wt = _dev(x), _dev(w)
+    off = torch.empty(rows * d + 1, device="cuda")[1:].view(rows, d)
+    off.copy_(xt)
+    for scale in (wt, None):
+        buf = torch.full((rows * d + 256,), 7.0, device="cuda")
+        y = zest_gpu.rms_norm(xt, 1e-6, scale, y=buf[:rows * d].view(rows, d))
+        got = _host(y)
+        assert np.array_equal(_host(zest_gpu.rms_norm(off, 1e-6, scale)).view(np.uint32), got.view(np.uint32))
+        assert bool((buf[rows * d:] == 7.0).all())
+        want = oracle.rms_norm(x, 1e-6)
+        want = oracle.mul_row(want, w) if scale is not None else want
+        fine = np.isfinite(x).all(axis=1)
+        assert nrmse(got[fine], want[fine]) <= EXACT
