@@ -95,11 +95,20 @@ struct gemm_cfg {
 };
 
 // LDS rows are 128 bytes = 8 chunks of 16 bytes (one block as bf16 each);
-// chunk c of row r is stored at position c ^ swz(r), with
-// swz(r) = (r % 8) ^ ((r / 8) % 2). Any 8 consecutive rows of one chunk
-// index then fall in 8 different 16-byte bank groups, and swz depends only on
-// r % 16, so the +32-row offsets of the MFMA tiles stay immediates.
-__device__ inline int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+// chunk c of row r is stored at position c ^ swz(r). swz is a linear map of
+// the low four bits b of r, (b0^b1^b2, b1, b2^b3), for which no access has a
+// bank conflict, whether 8 lanes meet in 128 bytes of banks or 16 in 256:
+//   * a fragment read (one chunk of consecutive rows): swz takes 8 values
+//     over 8 rows, and over the 8 even and the 8 odd rows of 16;
+//   * a producer's store of two lanes a row (chunks c and c ^ 4): swz % 4
+//     takes 4 values over 4 rows, and over the even and the odd rows of 8;
+//   * a one-unit producer's, four lanes a row (chunks c, c ^ 2, c ^ 4, c ^ 6):
+//     swz % 2 differs within two rows, and between rows r and r + 2.
+// It depends only on r % 16, so the +32-row offsets of the MFMA tiles stay
+// immediates.
+__device__ inline int swz(int row) {
+    return ((row ^ (row >> 1) ^ (row >> 2)) & 1) | (row & 2) | ((((row >> 2) ^ (row >> 3)) & 1) << 2);
+}
 
 __device__ inline void lds_put(uint8_t * smem, int off, uint4 v) { *reinterpret_cast<uint4 *>(smem + off) = v; }
 
@@ -126,13 +135,15 @@ typedef __attribute__((address_space(3))) void * lds_ptr_t;
 // vector offset. The hardware range check covers the vector offset only, so
 // every slab offset a load is given names a K-step of the operand (callers
 // clamp the steps past the end to the last one). With U = 2, thread p takes
-// two adjacent units of tile p/32 of the W slab: row p%16, column quarters 2h
-// and 2h+1 with h = p/16%2, i.e. 32 contiguous mantissa bytes (two 16-byte
+// two adjacent units of tile p/32 of the W slab: row p/2%16, column quarters
+// 2h and 2h+1 with h = p%2, i.e. 32 contiguous mantissa bytes (two 16-byte
 // loads) and 4 contiguous exponent bytes (one 4-byte load). With U = 1 (the
 // slab's last tiles, after the NP2/32 of the two-unit threads), thread p
-// takes one unit of tile NP2/32 + p/64: row p%16, quarter q = p/16%4 (16
-// mantissa bytes, 2 exponent bytes). 16 consecutive lanes are 16 consecutive
-// rows, for the swizzled stores.
+// takes one unit of tile NP2/32 + p/64: row p/4%16, quarter p%4 (16 mantissa
+// bytes, 2 exponent bytes). Consecutive lanes so take consecutive bytes of a
+// tile: the vector cache serves such loads at 64 B/clk a CU, and at 32 with
+// consecutive lanes on consecutive rows, 64 bytes apart (2048 x 7168 x 2560 in
+// one group 66 -> 64.8 us, 1024 x 2560 x 2560 alone 26 -> 25.3).
 template <class C, int U = 2>
 struct producer {
     static_assert(U == 1 || U == 2, "one or two W units a thread");
@@ -142,8 +153,8 @@ struct producer {
 
     __device__ producer(const uint8_t * W, int64_t w_bytes, int p) {
         rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W), (short) 0, (int) w_bytes, 0x00020000);
-        const int t = U == 2 ? p >> 5 : C::NP2 / 32 + (p >> 6), row = p & 15;
-        const int q0 = U == 2 ? 2 * ((p >> 4) & 1) : (p >> 4) & 3;  // the first unit's quarter
+        const int t = U == 2 ? p >> 5 : C::NP2 / 32 + (p >> 6), row = (U == 2 ? p >> 1 : p >> 2) & 15;
+        const int q0 = U == 2 ? 2 * (p & 1) : p & 3;  // the first unit's quarter
         vwm = t * ZEST_TILE_BYTES + row * ZEST_TILE_K + q0 * 16;
         vwe = t * ZEST_TILE_BYTES + ZEST_TILE_MANT + row * 8 + q0 * 2;
         const int wrow = t * 16 + row, sw = swz(wrow);
