@@ -175,14 +175,12 @@ struct producer {
         }
     }
 
-    // W unit i of a step, by the branch-free fast expansion, stored; true if
-    // the unit needs the general expansion (store_w_general) instead.
-    __device__ bool store_w_unit(const stage_regs<C, U> & st, int i, uint8_t * smem, int stage) const {
+    // W unit i of a step by the branch-free fast expansion, stored.
+    __device__ void store_w_unit(const stage_regs<C, U> & st, int i, zest::zest_u16x2 d, uint8_t * smem, int stage) const {
         uint32_t b[8];
-        const bool slow = zest::expand16_fast(st.wm[i], i ? st.we >> 16 : st.we & 0xffffu, b);
+        zest::expand16_by(st.wm[i], d, b);
         lds_put(smem, stw[i][0] + stage, make_uint4(b[0], b[1], b[2], b[3]));
         lds_put(smem, stw[i][1] + stage, make_uint4(b[4], b[5], b[6], b[7]));
-        return slow;
     }
 
     // Every unit of the step by the general expansion, stored.
@@ -196,14 +194,22 @@ struct producer {
         }
     }
 
-    // The units take the branch-free fast expansion; a unit whose exponent
-    // bytes need the general one is redone behind a single wave-uniform
-    // branch, which real weights almost never take.
+    // The units take the branch-free fast expansion; a step with a unit whose
+    // exponent bytes need the general one is redone behind a single
+    // wave-uniform branch, which real weights almost never take. Its condition
+    // is made first, so it is there long before the branch.
     __device__ void store_w(const stage_regs<C, U> & st, uint8_t * smem, int stage) const {
-        bool slow = false;
+        zest::zest_u16x2 d[U];
 #pragma unroll
-        for (int i = 0; i < U; i++) slow |= store_w_unit(st, i, smem, stage);
-        if (__builtin_expect(__any(slow), 0)) store_w_general(st, smem, stage);
+        for (int i = 0; i < U; i++) d[i] = zest::exp_offsets(st.we, i);
+        const bool general = zest::exp_general(U == 2 ? __builtin_elementwise_max(d[0], d[U - 1]) : d[0]);
+        const uint64_t any = __builtin_amdgcn_ballot_w64(general);
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            store_w_unit(st, i, d[i], smem, stage);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (__builtin_expect(any != 0, 0)) store_w_general(st, smem, stage);
     }
 };
 
@@ -569,23 +575,6 @@ __device__ inline void bare_barrier() {
 // (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 __device__ inline void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
-// One steady-state producer step: step j's W units (loaded two steps ago)
-// expanded and stored into `stage`, step j+2's requested into the same
-// registers. A unit whose exponent bytes need the general expansion is
-// redone behind one wave-uniform branch, which real weights almost never take.
-template <class C, int U>
-__device__ inline void produce_step(const producer<C, U> & pr, uint8_t * smem, int stage, stage_regs<C, U> & r,
-                                   int w_off_next) {
-    bool slow = false;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        slow |= pr.store_w_unit(r, u, smem, stage);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (__builtin_expect(__any(slow), 0)) pr.store_w_general(r, smem, stage);
-    pr.load_w(r, w_off_next);
-}
-
 // The producer's part of one tile over K-steps [k0, k0 + ns), with steps 0
 // and 1 already requested into r0 and r1: step j's W units are loaded during
 // step j-4 and stored into stage j%3 during step j-2 (the consumers read step
@@ -616,11 +605,13 @@ __device__ inline void produce_tile(const producer<C, U> & pr, uint8_t * smem, i
     // during step k: step k+2 stored into stage (k+2)%3, step k+4 requested
     int stage = 2 * C::STAGE, k = 0;
     for (; k + 5 < ns; k += 2) {
-        produce_step<C, U>(pr, smem, stage, r0, w0 + (k + 4) * w_kstride);
+        pr.store_w(r0, smem, stage);
+        pr.load_w(r0, w0 + (k + 4) * w_kstride);
         stage = stage == 2 * C::STAGE ? 0 : stage + C::STAGE;
         wait_lgkm0();
         bare_barrier();
-        produce_step<C, U>(pr, smem, stage, r1, w0 + (k + 5) * w_kstride);
+        pr.store_w(r1, smem, stage);
+        pr.load_w(r1, w0 + (k + 5) * w_kstride);
         stage = stage == 2 * C::STAGE ? 0 : stage + C::STAGE;
         wait_lgkm0();
         bare_barrier();

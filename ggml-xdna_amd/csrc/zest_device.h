@@ -131,15 +131,26 @@ typedef unsigned short zest_u16x2 __attribute__((ext_vector_type(2)));
 //   most 126, so the sign bit never borrows, and q = 0 saturates to 0.
 // Two ops per value. Other exponent bytes go through expand8.
 //
-// expand16_fast is that fast path alone, branch-free so it can be scheduled
-// between MFMAs; it returns true when the unit needs expand8 instead (its
-// output is then not the decoded values and must be replaced).
-__device__ inline bool expand16_fast(const uint4 & m, uint32_t e2, uint32_t out[8]) {
-    // (133 - e) << 7 for each block
-    const int32_t d0 = 133 * 128 - (int32_t) ((e2 & 0xffu) << 7);
-    const int32_t d1 = 133 * 128 - (int32_t) ((e2 >> 8) << 7);
-    const zest_u16x2 dv0 = {(unsigned short) d0, (unsigned short) d0};
-    const zest_u16x2 dv1 = {(unsigned short) d1, (unsigned short) d1};
+// expand16_by is that fast path alone, branch-free so it can be scheduled
+// between MFMAs, with its exponent offsets made beforehand: exp_offsets takes
+// the exponent bytes of two blocks (a unit) to (133 - e) << 7, two 16-bit
+// halves of one dword; exp_general says of such halves, together, whether any
+// exponent byte is outside 7..133 (its unit's output is then not the decoded
+// values and must be replaced by expand16's).
+__device__ inline zest_u16x2 exp_offsets(uint32_t e, int unit) {  // unit 0: bytes 0 and 1 of e, 1: bytes 2 and 3
+    const uint32_t b = __builtin_amdgcn_perm(0u, e, unit ? 0x0c030c02u : 0x0c010c00u);
+    const zest_u16x2 k = {133 * 128, 133 * 128};
+    return k - (__builtin_bit_cast(zest_u16x2, b) << (unsigned short) 7);
+}
+
+// exponent bytes 7..133 <=> 0 <= (133 - e) * 128 <= 126 * 128, as unsigned
+__device__ inline bool exp_general(zest_u16x2 d) {
+    const zest_u16x2 most = {126 * 128, 126 * 128};
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(d, most)) != 0u;
+}
+
+__device__ inline void expand16_by(const uint4 & m, zest_u16x2 d, uint32_t out[8]) {
+    const zest_u16x2 d0 = {d.x, d.x}, d1 = {d.y, d.y};
     const uint32_t w[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -147,11 +158,9 @@ __device__ inline bool expand16_fast(const uint4 & m, uint32_t e2, uint32_t out[
         const int sh = (i & 1) * 16;
         const float lo = (float) (int8_t) (wd >> sh), hi = (float) (int8_t) (wd >> (sh + 8));
         const uint32_t b = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-        const zest_u16x2 r = __builtin_elementwise_sub_sat(__builtin_bit_cast(zest_u16x2, b), i < 4 ? dv0 : dv1);
+        const zest_u16x2 r = __builtin_elementwise_sub_sat(__builtin_bit_cast(zest_u16x2, b), i < 4 ? d0 : d1);
         out[i] = __builtin_bit_cast(uint32_t, r);
     }
-    // exponent bytes 7..133 <=> 0 <= (133 - e) * 128 <= 126 * 128
-    return max((uint32_t) d0, (uint32_t) d1) > 126u * 128u;
 }
 
 __device__ inline void expand16(const uint4 & m, uint32_t e2, uint32_t out[8]) {
