@@ -85,6 +85,11 @@ struct gemm_cfg {
     // K-group g's ring at g * RING; after the K loop, the epilogue regions
     // of group 0's waves in [0, BM*BN*4) and group g's sums at g * BM*BN*4
     static constexpr size_t LDS_BYTES = KG * (RING > (size_t) BM * BN * 4 ? RING : (size_t) BM * BN * 4);
+    // a split-K launch: FIX partial tiles of the fixup at once, each
+    // consumer wave's share of partial i at i * BM*BN*4 (as K-group i's sums)
+    static constexpr size_t LDS_MAX = 163840 / MINB, TILE_BYTES = (size_t) BM * BN * 4;
+    static constexpr int FIX = LDS_MAX / TILE_BYTES < 4 ? (int) (LDS_MAX / TILE_BYTES) : 4;
+    static constexpr size_t LDS_SPLIT = LDS_BYTES > FIX * TILE_BYTES ? LDS_BYTES : FIX * TILE_BYTES;
     // a persistent launch: the GLU epilogue's staging (WM rows of 16 TJ + 4
     // floats a wave) above the ring
     static constexpr size_t LDS_APART = (size_t) STAGES * STAGE + (size_t) (NC / 64) * WM * (16 * TJ + 4) * 4;
@@ -485,9 +490,10 @@ __device__ inline int partial_off(int unit, int wave, int i, int j, int q, int l
 // counter. The order is fixed, so the result does not depend on arrival
 // order; since a + b == b + a exactly, a last wave of split S-1 or S-2 (the
 // usual case: splits run in that order) starts from its own sums in acc and
-// reads one partial fewer, others read their own back like the rest. Each
-// partial comes into the wave's own LDS region by LDS DMA (all of its loads
-// in flight at once, no registers held), then is added from there. LDS is
+// reads one partial fewer, others read their own back like the rest. Up to
+// C::FIX partials at a time come into the wave's own LDS regions by LDS DMA
+// (all of their loads in flight at once, no registers held; one round trip to
+// the coherent level each cost 0.9 us a split), then are added from there. LDS is
 // free: the K loop is over, and this workgroup has no other tile. Returns
 // true for the last wave, whose acc then holds the tile's sums. No wave
 // waits for another.
@@ -518,44 +524,52 @@ __device__ inline bool fixup(f32x16 (&acc)[C::TI][C::TJ], const gemm_params & p,
     old = __shfl(old, 0);
     asm volatile("" ::: "memory");
     if (old != (uint32_t) (S - 1)) return false;
-    uint8_t * region = smem + wave * (C::WM * C::WN * 4);
+    constexpr int REGION = C::WM * C::WN * 4, TILE = C::BM * C::BN * 4;
+    uint8_t * region = smem + wave * REGION;
     // acc already holds p[S-1] (split S-1) or its commuted first sum's other
     // operand (split S-2)
     const bool own = split >= S - 2;
-    for (int v = own ? 1 : 0; v < S; v++) {
-        // operand v of the sum is p[S-1-v], except that a split-S-2 wave's
-        // second operand is p[S-1] (its own sums stand in for p[S-2]). u is
-        // uniform but derived from the split, which the tile arithmetic can
-        // leave in a vector register, and a DMA's scalar offset taken from
-        // one costs a loop per load
-        const int u = __builtin_amdgcn_readfirstlane(own && v == 1 ? (split == S - 1 ? S - 2 : S - 1) : S - 1 - v);
-        const int base = partial_off<C>(u * T + t, wave, 0, 0, 0, 0);
+    for (int v0 = own ? 1 : 0; v0 < S; v0 += C::FIX) {
+        for (int v = v0; v < S && v < v0 + C::FIX; v++) {
+            // operand v of the sum is p[S-1-v], except that a split-S-2 wave's
+            // second operand is p[S-1] (its own sums stand in for p[S-2]). u is
+            // uniform but derived from the split, which the tile arithmetic can
+            // leave in a vector register, and a DMA's scalar offset taken from
+            // one costs a loop per load
+            const int u =
+                __builtin_amdgcn_readfirstlane(own && v == 1 ? (split == S - 1 ? S - 2 : S - 1) : S - 1 - v);
+            const int base = partial_off<C>(u * T + t, wave, 0, 0, 0, 0);
+            uint8_t * to = region + (v - v0) * TILE;
 #pragma unroll
-        for (int x = 0; x < PARTS; x++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr_t) (region + x * 1024), 16, lane * 16,
-                                                     base + x * 1024, 0, ZEST_SC1);
+            for (int x = 0; x < PARTS; x++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_ptr_t) (to + x * 1024), 16, lane * 16,
+                                                         base + x * 1024, 0, ZEST_SC1);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        for (int v = v0; v < S && v < v0 + C::FIX; v++) {
+            const uint8_t * from = region + (v - v0) * TILE;
 #pragma unroll
-        for (int i = 0; i < C::TI; i++)
+            for (int i = 0; i < C::TI; i++)
 #pragma unroll
-            for (int j = 0; j < C::TJ; j++)
+                for (int j = 0; j < C::TJ; j++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 x =
-                        *reinterpret_cast<const float4 *>(region + ((i * C::TJ + j) * 4 + q) * 1024 + lane * 16);
-                    if (v == 0) {
-                        acc[i][j][4 * q] = x.x;
-                        acc[i][j][4 * q + 1] = x.y;
-                        acc[i][j][4 * q + 2] = x.z;
-                        acc[i][j][4 * q + 3] = x.w;
-                    } else {
-                        acc[i][j][4 * q] += x.x;
-                        acc[i][j][4 * q + 1] += x.y;
-                        acc[i][j][4 * q + 2] += x.z;
-                        acc[i][j][4 * q + 3] += x.w;
+                    for (int q = 0; q < 4; q++) {
+                        const float4 x =
+                            *reinterpret_cast<const float4 *>(from + ((i * C::TJ + j) * 4 + q) * 1024 + lane * 16);
+                        if (v == 0) {
+                            acc[i][j][4 * q] = x.x;
+                            acc[i][j][4 * q + 1] = x.y;
+                            acc[i][j][4 * q + 2] = x.z;
+                            acc[i][j][4 * q + 3] = x.w;
+                        } else {
+                            acc[i][j][4 * q] += x.x;
+                            acc[i][j][4 * q + 1] += x.y;
+                            acc[i][j][4 * q + 2] += x.z;
+                            acc[i][j][4 * q + 3] += x.w;
+                        }
                     }
-                }
-        // the reads are done before the next partial's DMA overwrites them
+        }
+        // the reads are done before the next partials' DMA overwrites them
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     if (lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1066,98 +1080,54 @@ __global__ __launch_bounds__(CB::NT, 1) void gemm_kernel_mixed_tiles(const gemm_
     }
 }
 
-// 256x128 tiles (4 consumer waves of 64x128); 128x128 (4 of 32x128) where
-// the cost model prefers them (few rows, or too few big tiles).
-#ifndef ZEST_GEMM_BIG
-#define ZEST_GEMM_BIG 256, 128, 4
-#endif
-#ifndef ZEST_GEMM_SMALL
-#define ZEST_GEMM_SMALL 128, 128, 4
-#endif
-// Launch cost model, in K-steps of a 256x128 tile at full occupancy (about
-// 0.85 us): T tiles on P CUs take ceil(T/P) rounds of nk steps, plus PROLOGUE
-// steps per round to fill the pipeline. S K-splits take ceil(T*S/P) rounds of
-// nk/S steps, plus the fixup: every split writes its fp32 tile and the last
-// reads all S back through HBM, 2*T*S*BM*BN*4 bytes at about FIX_BW bytes
-// per step, and FIX_LAT steps more: the fixup's round trips (store and
-// acknowledge, count in, read back) that follow the K loop of every split
-// launch, however little data they move. A 128x128 step costs SMALL_STEP of
-// a 256x128 one (half the MFMA work, not half the waiting). The cheapest plan
-// wins.
 #ifndef ZEST_GEMM_PERSIST
 #define ZEST_GEMM_PERSIST 1
 #endif
 #ifndef ZEST_GEMM_MAX_SPLIT
 #define ZEST_GEMM_MAX_SPLIT 16
 #endif
-#ifndef ZEST_GEMM_PROLOGUE
-#define ZEST_GEMM_PROLOGUE 2.0
-#endif
-#ifndef ZEST_GEMM_FIX_BW
-#define ZEST_GEMM_FIX_BW 4.25e6  // bytes per step: ~5 TB/s x 0.85 us
-#endif
-#ifndef ZEST_GEMM_FIX_LAT
-#define ZEST_GEMM_FIX_LAT 5.0  // ~4 us
-#endif
-#ifndef ZEST_GEMM_SMALL_STEP
-#define ZEST_GEMM_SMALL_STEP 0.8
-#endif
-// 64x64 tiles (2 consumer waves of 32x64, 2 producers; two workgroups a CU)
-// for launches too small to fill the GPU with bigger tiles: a step of one
-// costs TINY_STEP of a 256x128 one, and two run on a CU side by side.
-#ifndef ZEST_GEMM_TINY
-#define ZEST_GEMM_TINY 64, 64, 2, 128, 2
-#endif
-#ifndef ZEST_GEMM_TINY_STEP
-#define ZEST_GEMM_TINY_STEP 0.45  // measured: ~0.38 us a step in a launch of 16 or 64 steps
-#endif
-// The same tiles as two K-groups (eight waves a workgroup), alone or with K
-// splits, for launches of at most one and a half such workgroups a CU: each
-// CU has twice the loads in flight, and the groups' sums meet in LDS instead
-// of through a split-K fixup in HBM (the down projection of a 1024-token
-// chunk at hidden 1024, 1024 x 1024 x 4096: 17.3 us against 21.3 in two
-// splits of single-group tiles; its O projection, K 1024: 8.1 against 9.2
-// unsplit). A group's step costs TINY2_STEP of a 256x128 one in the cost
-// model (fitted to the launch times of the hidden-1024 layer's four GEMMs at
-// 256 to 4096 tokens).
-#ifndef ZEST_GEMM_TINY2_STEP
-#define ZEST_GEMM_TINY2_STEP 0.4
-#endif
-// 256x128 tiles with 8 consumer waves of 32x128 and 4 producer waves, two
-// consumers on each SIMD: for the fused GLU (its long launches gain ~3% from
-// the second consumer), the whole tiles of mixed launches, and launches of
-// at most one round of whole tiles that 128x160 tiles cannot take (each CU
-// has one tile to hide its latencies in: the O projection at 2048 tokens as
-// 160 of these, 57.9 -> 55.7 us); other launches of several rounds lose what
-// the second consumer gains to its doubled W fragment reads.
-#ifndef ZEST_GEMM_GLU
-#define ZEST_GEMM_GLU 256, 128, 8, 256
-#endif
-// 128x160 tiles (4 consumer waves of 32x160) for a launch that 256x128 tiles
-// would run in one round, unsplit, when its weights are whole 160-row tiles
-// and these fit one round too: the O projection at 2048 tokens (2048 x 2560)
-// is 256 of them, one per CU, where 160 256x128 tiles leave 96 CUs idle
-// (55.5 -> ~49 us). The producers are this launch's critical path: four
-// waves take two W units a thread (tiles 0-7) and two waves one (tiles 8-9),
-// so the two SIMDs that hold a second producer wave carry one and a half
-// waves' expansion, not two (five waves of two units: 52.5 -> 48.6 us).
-// Launches with long K take them unsplit too when they fill more than half
-// the GPU (launch_any): the down projection (K 9728) at 2048 tokens, 96 us
-// against 104.5 us in three splits of 256x128 tiles.
-#ifndef ZEST_GEMM_O
-#define ZEST_GEMM_O 128, 160, 4, 384, 1, 1, 128
-#endif
-using cfg_big = gemm_cfg<ZEST_GEMM_BIG>;
-using cfg_o = gemm_cfg<ZEST_GEMM_O>;
-using cfg_small = gemm_cfg<ZEST_GEMM_SMALL>;
-using cfg_glu = gemm_cfg<ZEST_GEMM_GLU>;
-using cfg_tiny = gemm_cfg<ZEST_GEMM_TINY>;
+// The tile shapes. Which one a launch takes is the cost model's choice
+// (plan_plain, launch_any).
+//
+// 256x128 tiles: 4 consumer waves of 64x128, or 8 of 32x128, two on each SIMD
+// (the second hides latency that a CU with one tile in flight has nowhere else
+// to hide, for twice the reads of W fragments from LDS).
+using cfg_big = gemm_cfg<256, 128, 4>;
+using cfg_glu = gemm_cfg<256, 128, 8, 256>;
+// 128x160 tiles (4 consumer waves of 32x160) for weights of whole 160-row
+// tiles (the tiles then read only rows each packed weight holds): where 256x128
+// tiles leave CUs idle these may fill them (2048 x 2560 is 256 of them, one a CU, and
+// 160 of the others). The producers are their critical path: four waves take
+// two W units a thread (tiles 0-7) and two waves one (tiles 8-9), so the two
+// SIMDs that hold a second producer wave carry one and a half waves'
+// expansion, not two (five waves of two units: 52.5 -> 48.6 us).
+using cfg_o = gemm_cfg<128, 160, 4, 384, 1, 1, 128>;
+// The smaller tiles are bound by the chain of a producer's step (load, expand,
+// store, wait, barrier), not by the matrix cores: at 16 workgroups on an idle
+// GPU a K-step of a 128x128 tile took 0.38 us with producers of two units a
+// thread, 0.36 of them the producers alone and 0.24 the consumers alone. So
+// they have producers of one unit a thread, two waves on each SIMD whose
+// steps overlap, and 8 consumers where 4 would leave a SIMD's other wave to
+// wait for (128x128: 0.36 us; 1024 x 2560 x 2560 21.4 -> 20.0 us).
+using cfg_small = gemm_cfg<128, 128, 4, 512, 1, 2, 512>;
+// 128x64 tiles, two workgroups a CU (2048 x 1024 x 4096 31.6 -> 25.2 us, where
+// 64x64 tiles were the best before), and as two K-groups, one workgroup a CU,
+// for launches of up to one round of them: twice the loads in flight, and the
+// groups' sums meet in LDS, not through a split-K fixup in memory (768 x 2560 x
+// 4096 32.5 -> 22.4 us, 768 x 2560 x 2560 21.2 -> 15.0 us).
+using cfg_mid = gemm_cfg<128, 64, 4, 256, 2, 1, 256>;
+using cfg_mid2 = gemm_cfg<128, 64, 4, 256, 1, 1, 256, 2>;
+// 64x64 tiles as two K-groups, for fewer rows or columns still: one workgroup
+// a CU with producers of one unit a thread, or two with producers of two
+// (48 x 2560 x 2560 10.3 us with the second alone, 8.9 with the first in
+// two K splits; 48 x 19456 x 2560, 304 tiles, 20.9 with the first, 18.5 with the second).
+using cfg_tiny2 = gemm_cfg<64, 64, 2, 256, 1, 1, 256, 2>;
+using cfg_tiny2x2 = gemm_cfg<64, 64, 2, 128, 2, 1, 0, 2>;
 // Mixed launches run their whole tiles as cfg_glu's (two consumers per SIMD)
 // and the halves as 128x128 tiles of 8 consumer waves of 32x64 (4 row blocks
 // x 2 column blocks) and 4 producers, the same threads (the q/k/v group at
 // 2048 tokens: 66.8 -> 65.6 us against one consumer per SIMD in both).
 using cfg_half8 = gemm_cfg<128, 128, 4, 256, 1, 2>;
-using cfg_tiny2 = gemm_cfg<ZEST_GEMM_TINY, 1, 0, 2>;
 
 // Per device and stream: the split-K workspace (grown as needed; counters
 // zeroed when allocated, and zero again after every launch).
@@ -1245,7 +1215,8 @@ int set_lds(const char * name) {
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_kernel<C, EPI, SPLIT>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int) C::LDS_BYTES);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int) (SPLIT ? C::LDS_SPLIT : C::LDS_BYTES));
         if (e != hipSuccess) return zest::fail(ZEST_E_HIP, "%s: LDS attribute: %s", name, hipGetErrorString(e));
         attr_set.store(true, std::memory_order_release);
     }
@@ -1292,11 +1263,6 @@ int set_lds_mixed(const char * name) {
     return ZEST_OK;
 }
 
-struct gemm_plan {
-    int splits = 1;
-    double cost = 0;
-};
-
 // Tiles of a launch for one tile shape.
 int64_t tiles_of(const gemm_params & p, const int64_t * N, int BM, int BN) {
     int64_t nt = 0;
@@ -1304,26 +1270,49 @@ int64_t tiles_of(const gemm_params & p, const int64_t * N, int BM, int BN) {
     return ((p.M + BM - 1) / BM) * nt;
 }
 
-// The modelled cost of T tiles of nk steps on P CUs split S ways, with tiles
-// of tile_bytes fp32 and steps of `step` 256x128-steps.
-double split_cost(int64_t T, int nk, int64_t P, double tile_bytes, double step, int S) {
-    if (S == 1) return (double) ((T + P - 1) / P) * (nk + ZEST_GEMM_PROLOGUE) * step;
-    return (double) ((T * S + P - 1) / P) * ((double) nk / S + ZEST_GEMM_PROLOGUE) * step +
-           2.0 * T * S * tile_bytes / ZEST_GEMM_FIX_BW + ZEST_GEMM_FIX_LAT;
+// The launch cost model, in microseconds. U = T * S units (T tiles in S K
+// splits) on P CUs of `per_cu` workgroups each take whole rounds of P * per_cu
+// units and a last, partly filled one. A unit runs its K-steps (nk / (S * kg))
+// and `prologue` more (the pipeline's fill and the epilogue); a step takes
+// `step` with the GPU nearly idle and 1 + `load` times that when every CU
+// works (the clock falls under the power limit and the L2s fill up), rising
+// with the square of the share of CUs at work. A split launch pays for its partial sums:
+// each unit writes its tile and the last ones read them back, 2 * U * BM*BN*4
+// bytes at about 8 TB/s, and 0.75 us a split for their round trips. The
+// numbers are a least-squares fit, then a fit of the choice itself, to some
+// 6000 launches timed one plan after another: 18 weight shapes of hidden sizes 1024 to
+// 5120, 48 to 3000 rows. Over them the model's choice takes 0.7% longer than the best
+// plan measured for each, where the model before (rounds and steps of 256x128
+// tiles with constants for four shapes) took 7.3% longer than today's best.
+struct shape_rate {
+    int bm, bn, kg, per_cu, waves;  // waves: consumer waves, a counter each in a split launch
+    double fixed, prologue, step, load;
+};
+
+template <class C>
+constexpr shape_rate rate_of(double fixed, double prologue, double step, double load) {
+    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load};
 }
 
-// The cheapest number of K splits for T tiles (as split_cost).
-gemm_plan plan_splits(int64_t T, int nk, int64_t P, double tile_bytes, double step) {
-    gemm_plan best;
-    best.cost = split_cost(T, nk, P, tile_bytes, step, 1);
-    for (int S = 2; S <= ZEST_GEMM_MAX_SPLIT && nk / S >= 4; S++) {
-        const double cost = split_cost(T, nk, P, tile_bytes, step, S);
-        if (cost < best.cost) {
-            best.splits = S;
-            best.cost = cost;
-        }
-    }
-    return best;
+enum shape_kind { SHAPE_BIG, SHAPE_GLU, SHAPE_O, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2, SHAPES, SHAPE_MIXED };
+
+constexpr shape_rate RATES[SHAPES] = {
+    rate_of<cfg_big>(6.92, 4.53, 0.478, 0.610),     rate_of<cfg_glu>(4.36, 4.18, 0.487, 0.646),
+    rate_of<cfg_o>(4.95, 7.38, 0.370, 0.505),       rate_of<cfg_small>(3.10, 4.59, 0.347, 0.422),
+    rate_of<cfg_mid>(4.01, 0.97, 0.2475, 1.335),    rate_of<cfg_mid2>(2.68, 4.47, 0.371, 0.413),
+    rate_of<cfg_tiny2>(3.16, 3.56, 0.273, 0.236),   rate_of<cfg_tiny2x2>(4.30, 2.24, 0.323, 1.230),
+};
+
+// U units of `steps` K-steps, in rounds of `slots`
+double rounds_us(const shape_rate & r, int64_t U, double steps, int64_t slots) {
+    const double f = (double) (U % slots) / (double) slots, step = (steps + r.prologue) * r.step;
+    return (double) (U / slots) * step * (1 + r.load) + (U % slots ? step * (1 + r.load * f * f) : 0.0);
+}
+
+double plan_us(const shape_rate & r, int64_t T, int nk, int64_t P, int S) {
+    const int64_t U = T * S;
+    const double t = r.fixed + rounds_us(r, U, (double) nk / (S * r.kg), P * r.per_cu);
+    return S == 1 ? t : t + 0.75 * S + 2.0 * (double) U * r.bm * r.bn * 4 / 8e6;
 }
 
 // Plans and launches one GEMM (a group of weights, or the fused GLU). A
@@ -1386,7 +1375,7 @@ int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const ch
     const int st = p.splits > 1 ? set_lds<C, EPI, true>(name) : set_lds<C, EPI, false>(name);
     if (st != ZEST_OK) return st;
     if (p.splits > 1)
-        hipLaunchKernelGGL((gemm_kernel<C, EPI, true>), dim3((unsigned) grid), dim3(C::NT), C::LDS_BYTES, s, p);
+        hipLaunchKernelGGL((gemm_kernel<C, EPI, true>), dim3((unsigned) grid), dim3(C::NT), C::LDS_SPLIT, s, p);
     else
         hipLaunchKernelGGL((gemm_kernel<C, EPI, false>), dim3((unsigned) grid), dim3(C::NT), C::LDS_BYTES, s, p);
     return zest::check_launch(name);
@@ -1432,73 +1421,53 @@ int launch_mixed(gemm_params p, const int64_t * N, int64_t nbig, hipStream_t s, 
 }
 
 // The plan of a plain (or residual) launch: its tile shape and K splits.
-enum class shape_kind { o_round, mixed, tiny, small, o_one, glu_one, big };
 struct plain_plan {
-    shape_kind kind;
-    int splits;
-    int64_t nbig;  // mixed: the whole tiles
-    int kg = 1;    // tiny: K-groups
+    int kind = SHAPE_BIG;
+    int splits = 1;
+    int64_t nbig = 0;  // mixed: the whole tiles
+    double us = 1e300;
 };
 
-// The cost model above, applied: the cheapest of one round of 128x160 tiles
-// (long K), a mixed launch, 64x64 tiles (with their best K split, alone or as
-// two K-groups), 128x128 or 256x128 tiles (each with its best K split), and,
-// for one unsplit round, 128x160 or two-consumer 256x128 tiles.
+// The cheapest plan by the cost model: a tile shape with its K splits, or a
+// mixed launch. A launch whose whole tiles fill every CU is not split, a split
+// keeps at least three K-steps a K-group, and the partial sums of K up to 32768
+// fit the static workspace of zest_gemm_group_noalloc, which runs the same
+// plan (only a longer K is worth more: 2048 x 2816 x 65536 in four splits).
 plain_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P) {
-    const gemm_plan big =
-        plan_splits(tiles_of(p, N, cfg_big::BM, cfg_big::BN), p.nk, P, (double) cfg_big::BM * cfg_big::BN * 4, 1.0);
-    const gemm_plan small = plan_splits(tiles_of(p, N, cfg_small::BM, cfg_small::BN), p.nk, P,
-                                        (double) cfg_small::BM * cfg_small::BN * 4, ZEST_GEMM_SMALL_STEP);
+    plain_plan best;
     bool whole = true;  // every weight whole 160-row tiles
     for (int i = 0; i < p.nw; i++) whole &= N[i] % cfg_o::BN == 0;
-    const int64_t To = tiles_of(p, N, cfg_o::BM, cfg_o::BN);
-    // one round of 128x160 tiles, unsplit, when every weight is whole
-    // 160-row tiles, they fill more than half the GPU and K is long enough
-    // for the prologue not to matter: no split-K fixup traffic, and the
-    // tile's producers keep up with its consumers (the down projection at
-    // 2048 tokens, K 9728: 104.5 us in three splits, 96 us so)
-    if (whole && To <= P && 2 * To > P && p.nk >= 16) return {shape_kind::o_round, 1, 0};
-    // mixed: whole rounds of big tiles, the part-round left as half tiles
-    const int64_t Tb = tiles_of(p, N, cfg_big::BM, cfg_big::BN), R = Tb / P, rem = Tb - R * P;
+    for (int k = 0; k < SHAPES; k++) {
+        const shape_rate & r = RATES[k];
+        if (k == SHAPE_O && !whole) continue;
+        const int64_t T = tiles_of(p, N, r.bm, r.bn), slots = P * r.per_cu;
+        for (int S = 1; S <= ZEST_GEMM_MAX_SPLIT; S++) {
+            if (S > 1 && (T >= slots || T * S > 4 * slots || p.nk < 3 * S * r.kg)) break;
+            if (S > 1 && (p.nk <= 512 || whole) &&
+                (T * S * r.bm * r.bn * 4 > (int64_t) ZEST_NOALLOC_PARTIAL_BYTES || T * r.waves > ZEST_NOALLOC_COUNTERS))
+                break;
+            if (r.kg > 1 && (p.nk % (S * r.kg) || p.nk < 2 * S * r.kg)) continue;
+            const double us = plan_us(r, T, p.nk, P, S);
+            if (us < best.us) best = {k, S, 0, us};
+        }
+    }
+    // whole rounds of 256x128 tiles, the part-round left as half tiles (its
+    // launch has no gap between the two: measured 4% under the sum)
+    const int64_t T = tiles_of(p, N, cfg_glu::BM, cfg_glu::BN), R = T / P, rem = T % P;
     if (R >= 1 && rem > 0 && R * P % 8 == 0) {
-        const double mixed =
-            ((double) R + (double) ((2 * rem + P - 1) / P) * ZEST_GEMM_SMALL_STEP) * (p.nk + ZEST_GEMM_PROLOGUE);
-        if (mixed < big.cost && mixed < small.cost) return {shape_kind::mixed, 1, R * P};
+        const shape_rate & w = RATES[SHAPE_GLU];
+        const double us =
+            0.96 * (w.fixed + rounds_us(w, R * P, p.nk, P) + rounds_us(RATES[SHAPE_SMALL], 2 * rem, p.nk, P));
+        if (us < best.us) best = {SHAPE_MIXED, 1, R * P, us};
     }
-    // tiny tiles, cfg_tiny::MINB of them a CU
-    const int64_t Tt = tiles_of(p, N, cfg_tiny::BM, cfg_tiny::BN);
-    const gemm_plan tiny =
-        plan_splits(Tt, p.nk, P * cfg_tiny::MINB, (double) cfg_tiny::BM * cfg_tiny::BN * 4, ZEST_GEMM_TINY_STEP);
-    // as two K-groups: the launch's nk/2 group steps in S splits
-    gemm_plan tiny2;
-    tiny2.splits = 0;
-    for (int S = 1; S <= 8; S *= 2) {
-        if (p.nk % (2 * S) || p.nk / (2 * S) < 4 || 2 * Tt * S > 3 * P) continue;
-        const double cost = split_cost(Tt, p.nk / 2, P, (double) cfg_tiny::BM * cfg_tiny::BN * 4,
-                                       ZEST_GEMM_TINY2_STEP, S);
-        if (tiny2.splits == 0 || cost < tiny2.cost) tiny2 = {S, cost};
-    }
-    if (tiny2.splits > 0 && tiny2.cost < tiny.cost && tiny2.cost < big.cost && tiny2.cost < small.cost)
-        return {shape_kind::tiny, tiny2.splits, 0, 2};
-    if (tiny.cost < big.cost && tiny.cost < small.cost) return {shape_kind::tiny, tiny.splits, 0};
-    if (small.cost < big.cost) return {shape_kind::small, small.splits, 0};
-    if (big.splits == 1 && Tb <= P) {
-        // one round of whole tiles: as 128x160 tiles where the weights are
-        // whole 160-row tiles (the tiles then read only rows each packed
-        // weight holds) and they fit one round too, else with two consumers
-        // per SIMD
-        if (whole && To <= P) return {shape_kind::o_one, 1, 0};
-        return {shape_kind::glu_one, 1, 0};
-    }
-    return {shape_kind::big, big.splits, 0};
+    return best;
 }
 
 // Plans and launches a GEMM; `fixed` as for launch(). A fused GLU launch
 // splits K as the plain launch of its 2F columns would, in as many K-groups
 // (so its gate and up sums are that launch's, bit for bit: a sum depends on
 // the K-steps' partition and order, not on the tile shape), and takes the
-// cheaper of 256x128 and 128x128 tiles at that split (64x64 tiles for
-// K-groups).
+// cheapest of its tile shapes for that partition.
 template <int EPI>
 int launch_any(gemm_params p, const int64_t * N, hipStream_t s, const char * name,
                const sk_space * fixed = nullptr) {
@@ -1506,33 +1475,44 @@ int launch_any(gemm_params p, const int64_t * N, hipStream_t s, const char * nam
     (void) hipGetDevice(&dev);
     const int64_t P = cu_count(dev);
     const plain_plan pp = plan_plain(p, N, P);
+    const int S = pp.splits;
     if constexpr (EPI >= 0) {
-        const int S = pp.splits;
         // The tiles cover the output operand's K padding too: the columns of
         // 2F rounded up to 128 rows of the gate/up pair, whose rows past 2F
         // are zero blocks, so the h columns past F store the packer's zeros
         // (with 64-column tiles and F % 64 == 32 the last tile would end at F).
         const int64_t Nt = (N[0] + 127) / 128 * 128;
-        if (pp.kg == 2) return launch<cfg_tiny2, EPI>(p, &Nt, S, s, name, fixed);
-        const double big = split_cost(tiles_of(p, N, cfg_glu::BM, cfg_glu::BN), p.nk, P,
-                                      (double) cfg_glu::BM * cfg_glu::BN * 4, 1.0, S);
-        const double small = split_cost(tiles_of(p, N, cfg_small::BM, cfg_small::BN), p.nk, P,
-                                        (double) cfg_small::BM * cfg_small::BN * 4, ZEST_GEMM_SMALL_STEP, S);
-        if (small < big) return launch<cfg_small, EPI>(p, &Nt, S, s, name, fixed);
-        return launch<cfg_glu, EPI>(p, &Nt, S, s, name, fixed);
+        const int kg = pp.kind == SHAPE_MIXED ? 1 : RATES[pp.kind].kg;
+        int kind = SHAPES;
+        double least = 1e300;
+        for (const int k : {SHAPE_GLU, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2}) {
+            if (RATES[k].kg != kg) continue;
+            const double us = plan_us(RATES[k], tiles_of(p, &Nt, RATES[k].bm, RATES[k].bn), p.nk, P, S);
+            if (us < least) {
+                kind = k;
+                least = us;
+            }
+        }
+        switch (kind) {
+            case SHAPE_SMALL: return launch<cfg_small, EPI>(p, &Nt, S, s, name, fixed);
+            case SHAPE_MID: return launch<cfg_mid, EPI>(p, &Nt, S, s, name, fixed);
+            case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, &Nt, S, s, name, fixed);
+            case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, &Nt, S, s, name, fixed);
+            case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, &Nt, S, s, name, fixed);
+            default: return launch<cfg_glu, EPI>(p, &Nt, S, s, name, fixed);
+        }
     } else {
         switch (pp.kind) {
-            case shape_kind::o_round:
-            case shape_kind::o_one: return launch<cfg_o, EPI>(p, N, 1, s, name, fixed);
-            case shape_kind::mixed: return launch_mixed<cfg_glu, cfg_half8, EPI>(p, N, pp.nbig, s, name);
-            case shape_kind::tiny:
-                if (pp.kg == 2) return launch<cfg_tiny2, EPI>(p, N, pp.splits, s, name, fixed);
-                return launch<cfg_tiny, EPI>(p, N, pp.splits, s, name, fixed);
-            case shape_kind::small: return launch<cfg_small, EPI>(p, N, pp.splits, s, name, fixed);
-            case shape_kind::glu_one: return launch<cfg_glu, EPI>(p, N, 1, s, name, fixed);
-            case shape_kind::big: break;
+            case SHAPE_GLU: return launch<cfg_glu, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_O: return launch<cfg_o, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_SMALL: return launch<cfg_small, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_MID: return launch<cfg_mid, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, N, S, s, name, fixed);
+            case SHAPE_MIXED: return launch_mixed<cfg_glu, cfg_half8, EPI>(p, N, pp.nbig, s, name);
+            default: return launch<cfg_big, EPI>(p, N, S, s, name, fixed);
         }
-        return launch<cfg_big, EPI>(p, N, pp.splits, s, name, fixed);
     }
 }
 

@@ -165,6 +165,63 @@ def test_scalar_offsets_stay_inside_operands(M, N, K):
         check_launch(M, N, K, 128, 160, 4, 1)
 
 
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_small_tile_shapes_stay_inside_operands(M, N, K):
+    # cfg_mid, and cfg_mid2, cfg_tiny2 and cfg_tiny2x2 as two K-groups, in
+    # every split the planner can give them (three steps a K-group at least);
+    # cfg_small's rows (4 row blocks, two column blocks); cfg_o in K splits
+    nk = k_steps(K)
+    for S in range(1, 17):
+        if S == 1 or nk >= 3 * S:
+            check_launch(M, N, K, 128, 64, 4, S)
+            check_launch(M, N, K, 128, 128, 4, S)
+            if N % 160 == 0:
+                check_launch(M, N, K, 128, 160, 4, S)
+        if nk % (2 * S) == 0 and nk >= (2 if S == 1 else 6 * S):
+            check_launch(M, N, K, 128, 64, 4, S, KG=2)
+            check_launch(M, N, K, 64, 64, 2, S, KG=2)
+
+
+# (BM, BN, consumer waves across rows, across columns, K-groups, workgroups a CU)
+LDS_SHAPES = [(256, 128, 4, 1, 1, 1), (256, 128, 8, 1, 1, 1), (128, 160, 4, 1, 1, 1), (128, 128, 4, 2, 1, 1),
+              (128, 64, 4, 1, 1, 2), (128, 64, 4, 1, 2, 1), (64, 64, 2, 1, 2, 1), (64, 64, 2, 1, 2, 2)]
+
+
+@pytest.mark.parametrize("BM,BN,CWM,CWN,KG,MINB", LDS_SHAPES)
+def test_split_fixup_lds_regions(BM, BN, CWM, CWN, KG, MINB):
+    # a split launch's LDS (LDS_SPLIT): FIX partial tiles at a time, wave w's
+    # share of the i-th at i*BM*BN*4 + w*WM*WN*4, its pieces of 1 KB inside
+    # it; every share apart, all inside the allocation, and MINB such
+    # workgroups in a CU's 160 KB
+    WM, WN, waves, tile, ring = BM // CWM, BN // CWN, CWM * CWN, BM * BN * 4, 3 * BN * 128
+    most = 163840 // MINB
+    fix = min(most // tile, 4)
+    lds = max(KG * max(ring, tile), fix * tile)
+    assert fix >= 1 and lds * MINB <= 160 * 1024
+    pieces = (WM // 32) * (WN // 32) * 4
+    assert pieces * 1024 == WM * WN * 4
+    shares = sorted((i * tile + w * WM * WN * 4, i * tile + (w + 1) * WM * WN * 4) for i in range(fix) for w in range(waves))
+    assert shares[0][0] == 0 and shares[-1][1] <= lds
+    assert all(a[1] <= b[0] for a, b in zip(shares, shares[1:]))
+
+
+@pytest.mark.parametrize("S", [2, 3, 4, 5, 16])
+@pytest.mark.parametrize("FIX", [1, 2, 3, 4])
+def test_split_fixup_sums_in_split_order(S, FIX):
+    # whichever split's wave arrives last, the sum is ((p[S-1] + p[S-2]) +
+    # p[S-3]) + ... + p[0], its first addition perhaps commuted (a wave of
+    # split S-1 or S-2 starts from its own sums)
+    for split in range(S):
+        own = split >= S - 2
+        order = [split] if own else []
+        v0 = 1 if own else 0
+        while v0 < S:
+            batch = range(v0, min(S, v0 + FIX))
+            order += [(S - 2 if split == S - 1 else S - 1) if own and v == 1 else S - 1 - v for v in batch]
+            v0 += FIX
+        assert sorted(order[:2]) == [S - 2, S - 1] and order[2:] == list(range(S - 3, -1, -1)), (split, order)
+
+
 def test_o_tiles_need_whole_160_row_weights():
     # the launch rule has teeth: 160-row tiles over a weight of 200 rows
     # would read rows its packed operand (256 rows) does not hold

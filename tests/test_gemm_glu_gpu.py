@@ -158,6 +158,24 @@ def test_gemm_glu_bit_exact_order_sensitive(zest_gpu, M, F, K):
 
 
 @pytest.mark.parametrize("M,F,K", [
+    (300, 1664, 1536),   # 128x64 tiles in two K-groups
+    (300, 2720, 1280),   # the plain launch so, the fused one as 64x64 tiles, two workgroups a CU
+    (600, 800, 1280),    # the plain launch as 64x64 tiles, the fused one as 128x64, both two K-groups
+    (129, 96, 2560),     # 64x64 tiles in two K-groups and two K splits
+    (129, 32, 3072),     # and three
+    (129, 2592, 64),     # 128x64 tiles of one K-step
+    (600, 1024, 3080),   # an odd number of K-steps: no K-groups
+    (1000, 1760, 1280),  # the plain launch as 128x64 tiles, the fused one as 128x128
+    (600, 2880, 1536),   # 128x128 tiles, 16 waves
+    (600, 3520, 1536),   # the plain launch as 128x160 tiles, the fused one as 256x128
+])
+def test_gemm_glu_planned_shapes(zest_gpu, M, F, K):
+    """The fused launch's tile shapes give the plain launch's sums whatever shape that one takes."""
+    test_gemm_glu_bit_exact_order_sensitive(zest_gpu, M, F, K)
+    test_gemm_glu_writes_the_operand_padding(zest_gpu, M, F, K)
+
+
+@pytest.mark.parametrize("M,F,K", [
     (65, 96, 2560),     # 64x64 tiles in K-groups and K splits; F % 64 == 32
     (300, 96, 200),     # 128-column tiles; F % 64 == 32
     (1024, 160, 4096),  # 64x64 tiles in K-groups; F % 64 == 32

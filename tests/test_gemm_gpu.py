@@ -109,6 +109,57 @@ def test_gemm_against_oracle(zest_gpu, oracle, wtype, M, N, K):
     assert maxrel32 <= 1e-3
 
 
+@pytest.mark.parametrize("M,ns,K", [
+    (777, [2050], 1000),            # 128x64 tiles in two K-groups; ragged rows, columns and K
+    (200, [2050], 5120),            # and in two K splits
+    (129, [64], 64),                # one K-step, 128x64 tiles
+    (1000, [1119], 3208),           # 128x64 tiles, two a CU, an odd number of K-steps
+    (511, [1600], 4104),            # in three K splits
+    (129, [200], 4104),             # in four: two rounds of the fixup
+    (1300, [2400], 3072),           # 128x128 tiles, 16 waves
+    (100, [1000], 2560),            # 64x64 tiles in two K-groups and two K splits
+    (777, [96], 3072),              # and three
+    (33, [200], 5120),              # and four
+    (48, [9728, 9728], 2560),       # 304 of them, two workgroups a CU
+    (511, [3000], 5120),            # 128x64 tiles in two K-groups, 188 of them
+    (1300, [3000], 1280),           # 256x128 tiles, 8 consumers
+    (300, [800, 160, 35], 1024),    # a group
+    (768, [2560], 17408),           # 256x128 tiles in four K splits
+])
+def test_gemm_planned_shapes(zest_gpu, oracle, M, ns, K):
+    """Every tile shape of the planner at ragged edges, with the K splits and K-groups it gives them, against fp64
+    on the first, last and sampled rows (the bound of two roundings a product term of gemm_check); the residual
+    form is the plain one plus the add, bit for bit; nothing outside the output's columns is written."""
+    import torch
+    x = Rng(M + sum(ns)).normal(M * K).reshape(M, K)
+    a = zest_gpu.pack_act_x(torch.from_numpy(x).cuda())
+    rows = np.unique(np.concatenate([[0, M - 1], np.linspace(0, M - 1, 24).astype(int)]))
+    ad = decoded_act(zest_gpu, oracle, a, M, K)[rows]
+    ws, outs = [], []
+    for i, n in enumerate(ns):
+        w = Rng(M + K + i).normal(n * K, 0, 0.02).reshape(n, K)
+        ws.append(zest_gpu.convert_weight(0, torch.from_numpy(w).cuda().view(torch.uint8), n, K))
+        outs.append(torch.full((M, n + 5), 7.0, device="cuda"))
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    zest_gpu.gemm_group(a, M, ws, ns, K, outs=outs, nonfinite=flag)
+    again = [torch.zeros_like(o) for o in outs]
+    zest_gpu.gemm_group(a, M, ws, ns, K, outs=again, nonfinite=flag)
+    torch.cuda.synchronize()
+    assert int(flag[0]) == 0
+    for n, w, o, o2 in zip(ns, ws, outs, again):
+        assert torch.equal(o[:, :n], o2[:, :n])
+        assert bool((o[:, n:] == 7.0).all())
+        r64, ab = oracle.mul_mat_f64(decoded(zest_gpu, oracle, w, n, K), ad)
+        worst, maxrel = gemm_check(o.cpu().numpy()[rows][:, :n], r64, ab, K)
+        assert worst <= 1.0 and maxrel <= 1e-3, (worst, maxrel)
+    if len(ns) == 1 and ns[0] % 4 == 0:
+        n = ns[0]
+        res = torch.randn((M, n), device="cuda")
+        got = zest_gpu.gemm_residual(a, M, ws[0], n, K, res)
+        torch.cuda.synchronize()
+        assert torch.equal(got, outs[0][:, :n] + res)
+
+
 def test_gemm_full_size_ffn_properties(zest_gpu, oracle):
     # BASELINE config 2 sizes: gate 2048 x 9728 x 2560 with 1% outlier
     # channels; checked on sampled rows, plus linearity in the activations

@@ -137,3 +137,30 @@ def test_noalloc_under_graph_capture(zest_gpu):
         # eager work on the same array between replays
         z.gemm_group(a, 600, ws, ns, K, outs=[torch.empty((600, ns[0]), device="cuda")], noalloc=True)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 2050, 5120), (129, 200, 4104), (33, 200, 5120)])
+def test_noalloc_split_plans_under_capture(zest_gpu, M, N, K):
+    """Plans in two to four K splits (128x64 tiles in K-groups and alone, 64x64 tiles), captured and replayed with
+    eager calls on the same array between: every replay gives the allocating call's bits."""
+    import torch
+    z = zest_gpu
+    a, ws = _case(z, M, [N], K, 7)
+    want = z.gemm_group(a, M, ws, [N], K)[0].clone()
+    out = torch.empty((M, N), device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        z.gemm_group(a, M, ws, [N], K, outs=[out], noalloc=True)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        z.gemm_group(a, M, ws, [N], K, outs=[out], noalloc=True)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+        z.gemm_group(a, M, ws, [N], K, outs=[torch.empty((M, N), device="cuda")], noalloc=True)
+        torch.cuda.synchronize()
