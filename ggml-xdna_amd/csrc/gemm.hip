@@ -30,6 +30,7 @@
 #include <mutex>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "zest_common.h"
 #include "zest_device.h"
@@ -1130,12 +1131,16 @@ using cfg_tiny2x2 = gemm_cfg<64, 64, 2, 128, 2, 1, 0, 2>;
 using cfg_half8 = gemm_cfg<128, 128, 4, 256, 1, 2>;
 
 // Per device and stream: the split-K workspace (grown as needed; counters
-// zeroed when allocated, and zero again after every launch).
+// zeroed when allocated, and zero again after every launch). Buffers that a
+// captured graph names are not freed when they are outgrown, as the graph may
+// be replayed: `held` keeps them until zest_release_stream.
 struct sk_space {
     float * partial = nullptr;
     size_t partial_bytes = 0;
     uint32_t * counters = nullptr;
     size_t n_counters = 0;
+    bool captured = false;
+    std::vector<void *> held;
 };
 
 // Clears n counters (a kernel, not a memset, so a captured graph replays it).
@@ -1178,15 +1183,37 @@ int cu_count(int dev) {
 std::mutex g_sk_mu;
 std::map<std::pair<int, hipStream_t>, sk_space> g_sk_spaces;
 
+// A split-K workspace of at least these sizes, in `out`. Nothing can be
+// allocated while the stream is being captured: there `out.partial` is null
+// where the stream's workspace is too small (the launch then runs unsplit).
 int sk_reserve(hipStream_t s, size_t partial_bytes, size_t n_counters, sk_space & out, const char * name) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return zest::fail(ZEST_E_HIP, "%s: hipGetDevice failed", name);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &capture) != hipSuccess)
+        return zest::fail(ZEST_E_HIP, "%s: hipStreamIsCapturing failed", name);
     std::lock_guard<std::mutex> lock(g_sk_mu);
     sk_space & sp = g_sk_spaces[{dev, s}];
+    const bool fits = sp.partial_bytes >= partial_bytes && sp.n_counters >= n_counters;
+    out.partial = nullptr;
+    if (capture != hipStreamCaptureStatusNone) {
+        if (!fits) return ZEST_OK;
+        sp.captured = true;
+    }
     // a launch still running on the stream may use the buffers being replaced
-    if ((sp.partial_bytes < partial_bytes || sp.n_counters < n_counters) && (sp.partial || sp.counters) &&
-        hipStreamSynchronize(s) != hipSuccess)
+    if (!fits && (sp.partial || sp.counters) && hipStreamSynchronize(s) != hipSuccess)
         return zest::fail(ZEST_E_HIP, "%s: stream synchronize", name);
+    if (!fits && sp.captured) {
+        for (void * b : {(void *) sp.partial, (void *) sp.counters})
+            if (b) sp.held.push_back(b);
+        // both anew, and at least twice the size, so few are ever held
+        partial_bytes = std::max(partial_bytes, 2 * sp.partial_bytes);
+        n_counters = std::max(n_counters, 2 * sp.n_counters);
+        sp.partial = nullptr;
+        sp.counters = nullptr;
+        sp.partial_bytes = sp.n_counters = 0;
+        sp.captured = false;
+    }
     if (sp.partial_bytes < partial_bytes) {
         if (sp.partial) (void) hipFree(sp.partial);
         sp.partial = nullptr;
@@ -1204,7 +1231,10 @@ int sk_reserve(hipStream_t s, size_t partial_bytes, size_t n_counters, sk_space 
             return zest::fail(ZEST_E_HIP, "%s: split-K counters", name);
         sp.n_counters = n;
     }
-    out = sp;
+    out.partial = sp.partial;
+    out.partial_bytes = sp.partial_bytes;
+    out.counters = sp.counters;
+    out.n_counters = sp.n_counters;
     return ZEST_OK;
 }
 
@@ -1352,6 +1382,8 @@ int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const ch
         } else {
             const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
             if (st != ZEST_OK) return st;
+            // under capture, on a stream that no such launch has run on yet
+            if (!sp.partial) return launch<C, EPI>(p, N, 1, s, name);
         }
         p.partial = sp.partial;
         p.counters = sp.counters;
@@ -1649,6 +1681,7 @@ extern "C" int zest_release_stream(void * stream) {
         synced = true;
         if (it->second.partial) (void) hipFree(it->second.partial);
         if (it->second.counters) (void) hipFree(it->second.counters);
+        for (void * b : it->second.held) (void) hipFree(b);
         it = g_sk_spaces.erase(it);
     }
     return ZEST_OK;

@@ -149,7 +149,12 @@ ZEST_API int zest_gemm_residual(const void *a, int64_t M, const void *w, int64_t
  * tile's K among workgroups (split-K) and sums the splits in a fixed order,
  * through a workspace the library allocates per device and stream on first
  * use (and grows, synchronizing the stream; zest_release_stream frees it):
- * calls that share a stream run in order and never share it concurrently. A launch of at most one small
+ * calls that share a stream run in order and never share it concurrently.
+ * Under stream capture nothing is allocated: a launch whose stream does not
+ * hold a large enough workspace yet runs unsplit, and one that a graph was
+ * captured with is kept until zest_release_stream, also when a later call
+ * outgrows it (a replay uses it, so replays must not overlap calls on the
+ * stream it was captured on). A launch of at most one small
  * tile a CU may instead split each tile's K between two groups of waves in
  * one workgroup (K-groups), whose sums meet in LDS, also in a fixed order.
  * The same holds for zest_gemm and zest_gemm_glu, which run through the

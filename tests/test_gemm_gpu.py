@@ -625,3 +625,45 @@ def test_release_stream_frees_and_regrows_the_split_k_workspace(zest_gpu, oracle
     r64, ab = oracle.mul_mat_f64(decoded(zest_gpu, oracle, wp, N, K), decoded_act(zest_gpu, oracle, a, M, K)[rows])
     worst, _ = gemm_check(c0[rows], r64, ab, K)
     assert worst <= 1.0
+
+
+def test_split_k_under_capture(zest_gpu, oracle):
+    """The allocating call captured on a stream that holds no workspace (it runs unsplit), then on one that does, with
+    the workspace outgrown between the replays: each replay within the bound, the second graph's the eager bits."""
+    import torch
+    M, N, K = 64, 512, 16384
+    z = zest_gpu
+    a = z.pack_act_x(_dev(wide_blocks(1024, K, 5)))
+    small = z.pack_act_x(_dev(wide_blocks(M, K, 5)))
+    wp = z.convert_weight(0, _dev(wide_blocks(N, K, 6, 0.02).view(np.uint8)), N, K)
+    out, big = torch.empty((M, N), device="cuda"), torch.empty((1024, N), device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    rows = np.arange(0, M, 7)
+    r64, ab = oracle.mul_mat_f64(decoded(z, oracle, wp, N, K), decoded_act(z, oracle, small, M, K)[rows])
+    want = None
+    for warm in (False, True):
+        if warm:
+            with torch.cuda.stream(s):
+                z.gemm(small, M, wp, N, K, out=out)
+            s.synchronize()
+            want = out.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            z.gemm(small, M, wp, N, K, out=out)
+        torch.cuda.synchronize()
+        for rep in range(3):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            if warm:
+                assert torch.equal(out.view(torch.int32), want.view(torch.int32)), rep
+            else:
+                assert gemm_check(out.cpu().numpy()[rows], r64, ab, K)[0] <= 1.0, rep
+            if warm and rep == 0:
+                with torch.cuda.stream(s):
+                    z.gemm(a, 1024, wp, N, K, out=big)
+                s.synchronize()
+        del g
+    assert z.lib().zest_release_stream(s.cuda_stream) == 0
