@@ -54,6 +54,31 @@ def test_glu_split(zest_gpu, oracle, kind):
     assert nrmse(got, oracle.glu(kind, g, u)) <= EXACT
 
 
+@pytest.mark.parametrize("rows,f,stride,shift", [(1, 8, 8, 0), (15, 264, 264, 0), (17, 1000, 1003, 0), (33, 256, 260, 1), (257, 72, 80, 4)])
+def test_glu_edges(zest_gpu, oracle, rows, f, stride, shift):
+    """Rows and columns around the workgroup's 16 x 256, strides and starts that are not whole 16-byte pieces: the fp32
+    result against the oracle, its pack the packer's, padding rows and columns zero."""
+    import torch
+    g = Rng(71).normal(rows * f, 0, 1.5).reshape(rows, f)
+    u = Rng(72).normal(rows * f, 0, 1.5).reshape(rows, f)
+    views = []
+    for v in (g, u):
+        buf = torch.full((rows * stride + shift,), float("nan"), device="cuda")
+        views.append(buf[shift:].view(rows, stride)[:, :f])
+        views[-1].copy_(_dev(v))
+    packed = zest_gpu.empty_act(rows, f)
+    packed.view(torch.uint8).fill_(255)
+    got = _host(zest_gpu.glu(1, *views, f, packed=packed))
+    assert nrmse(got, oracle.glu(1, g, u)) <= EXACT
+    want = zest_gpu.pack_act_x(_dev(got))
+    assert torch.equal(packed.view(torch.uint8), want.view(torch.uint8))
+    # the fp32 result and the pack alone are the same bits
+    assert np.array_equal(_host(zest_gpu.glu(1, *views, f)).view(np.uint32), got.view(np.uint32))
+    packed.view(torch.uint8).fill_(255)
+    zest_gpu.glu(1, *views, f, y=None, packed=packed)
+    assert torch.equal(packed.view(torch.uint8), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("swapped", [False, True])
 def test_swiglu_one_tensor_and_fused_pack(zest_gpu, oracle, swapped):
     # one tensor [rows][2f]: gate and up are its halves (swapped: up first)
