@@ -1304,39 +1304,54 @@ int64_t tiles_of(const gemm_params & p, const int64_t * N, int BM, int BN) {
 // splits) on P CUs of `per_cu` workgroups each take whole rounds of P * per_cu
 // units and a last, partly filled one. A unit runs its K-steps (nk / (S * kg))
 // and `prologue` more (the pipeline's fill and the epilogue); a step takes
-// `step` with the GPU nearly idle and 1 + `load` times that when every CU
-// works (the clock falls under the power limit and the L2s fill up), rising
-// with the square of the share of CUs at work. A split launch pays for its partial sums:
-// each unit writes its tile and the last ones read them back, 2 * U * BM*BN*4
-// bytes at about 8 TB/s, and 0.75 us a split for their round trips. The
-// numbers are a least-squares fit, then a fit of the choice itself, to some
-// 6000 launches timed one plan after another: 18 weight shapes of hidden sizes 1024 to
-// 5120, 48 to 3000 rows. Over them the model's choice takes 0.7% longer than the best
-// plan measured for each, where the model before (rounds and steps of 256x128
-// tiles with constants for four shapes) took 7.3% longer than today's best.
+// `step` with the GPU nearly idle and `full` times that in a whole round (the
+// clock falls under the power limit and the L2s fill up). In between it rises
+// with the square of the share of CUs at work; where two workgroups fit a CU, to
+// 1 + `load` with one on each, then, once any CU has two, on a line from `pair`
+// to `full` (128x64 tiles, a step's time over one workgroup's: 1.6 with 1.1 a CU,
+// 2.0 with 2). A split launch pays for its partial sums: each unit writes its tile
+// and the last ones read them back, 2 * U * BM*BN*4 bytes at about 8 TB/s, and
+// 0.75 us a split for their round trips. The numbers are a fit of the choice
+// itself to some 6000 launches timed one plan after another (18 weight shapes of
+// hidden sizes 1024 to 5120, 48 to 3000 rows), then to 957 launches with all
+// their plans over all widths and 32 to 4096 rows, the fused and the residual
+// ones among them: over these the choice takes 0.4% longer than the best plan
+// measured for each, where the first fit, which had a square of the share for
+// two workgroups a CU as well, took 1.0% (773 x 2816 x 11008 with 1.2 such
+// workgroups a CU 79 us, its best plan 63).
 struct shape_rate {
     int bm, bn, kg, per_cu, waves;  // waves: consumer waves, a counter each in a split launch
-    double fixed, prologue, step, load;
+    double fixed, prologue, step, load, pair, full;
 };
 
 template <class C>
 constexpr shape_rate rate_of(double fixed, double prologue, double step, double load) {
-    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load};
+    static_assert(C::MINB == 1, "one workgroup a CU");
+    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load, 0.0, 1 + load};
+}
+
+template <class C>
+constexpr shape_rate rate_of(double fixed, double prologue, double step, double load, double pair, double full) {
+    static_assert(C::MINB == 2, "two workgroups a CU");
+    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load, pair, full};
 }
 
 enum shape_kind { SHAPE_BIG, SHAPE_GLU, SHAPE_O, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2, SHAPES, SHAPE_MIXED };
 
 constexpr shape_rate RATES[SHAPES] = {
-    rate_of<cfg_big>(6.92, 4.53, 0.478, 0.610),     rate_of<cfg_glu>(4.36, 4.18, 0.487, 0.646),
-    rate_of<cfg_o>(4.95, 7.38, 0.370, 0.505),       rate_of<cfg_small>(3.10, 4.59, 0.347, 0.422),
-    rate_of<cfg_mid>(4.01, 0.97, 0.2475, 1.335),    rate_of<cfg_mid2>(2.68, 4.47, 0.371, 0.413),
-    rate_of<cfg_tiny2>(3.16, 3.56, 0.273, 0.236),   rate_of<cfg_tiny2x2>(4.30, 2.24, 0.323, 1.230),
+    rate_of<cfg_big>(8.45, 4.53, 0.455, 0.470),    rate_of<cfg_glu>(5.34, 4.18, 0.455, 0.553),
+    rate_of<cfg_o>(3.87, 7.38, 0.353, 0.475),      rate_of<cfg_small>(2.68, 4.59, 0.391, 0.456),
+    rate_of<cfg_mid>(2.54, 7.26, 0.222, 0.294, 1.642, 1.929), rate_of<cfg_mid2>(2.72, 4.47, 0.350, 0.343),
+    rate_of<cfg_tiny2>(2.90, 3.56, 0.2795, 0.233), rate_of<cfg_tiny2x2>(2.64, 5.94, 0.305, 0.216, 1.675, 1.817),
 };
 
 // U units of `steps` K-steps, in rounds of `slots`
 double rounds_us(const shape_rate & r, int64_t U, double steps, int64_t slots) {
     const double f = (double) (U % slots) / (double) slots, step = (steps + r.prologue) * r.step;
-    return (double) (U / slots) * step * (1 + r.load) + (U % slots ? step * (1 + r.load * f * f) : 0.0);
+    double last = 0.0;  // the last, partly filled round
+    if (U % slots && r.per_cu == 1) last = 1 + r.load * f * f;
+    else if (U % slots) last = 2 * f <= 1 ? 1 + r.load * 4 * f * f : r.pair + (r.full - r.pair) * (2 * f - 1);
+    return step * ((double) (U / slots) * r.full + last);
 }
 
 double plan_us(const shape_rate & r, int64_t T, int nk, int64_t P, int S) {
