@@ -203,7 +203,13 @@ struct producer {
     // The units take the branch-free fast expansion; a step with a unit whose
     // exponent bytes need the general one is redone behind a single
     // wave-uniform branch, which real weights almost never take. Its condition
-    // is made first, so it is there long before the branch.
+    // is made first, so it is there long before the branch. Zero blocks (byte
+    // 0: the padding rows past N, the padding columns past K) come through it
+    // too, but a zero mantissa is zero whatever its exponent, so only units
+    // with a nonzero one are redone: else every step of the tiles that reach
+    // past N would be, and a launch takes as long as its slowest tile (1884 x
+    // 2316 x 11808 179 -> 106 us, 512 x 32001 x 4096 123 -> 108; 2304 and 32000
+    // columns take 103 and 104).
     __device__ void store_w(const stage_regs<C, U> & st, uint8_t * smem, int stage) const {
         zest::zest_u16x2 d[U];
 #pragma unroll
@@ -215,7 +221,13 @@ struct producer {
             store_w_unit(st, i, d[i], smem, stage);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (__builtin_expect(any != 0, 0)) store_w_general(st, smem, stage);
+        if (__builtin_expect(any != 0, 0)) {
+            bool redo = false;
+#pragma unroll
+            for (int i = 0; i < U; i++)
+                redo |= zest::exp_general(d[i]) && (st.wm[i].x | st.wm[i].y | st.wm[i].z | st.wm[i].w) != 0u;
+            if (__builtin_amdgcn_ballot_w64(redo)) store_w_general(st, smem, stage);
+        }
     }
 };
 

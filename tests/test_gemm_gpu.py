@@ -77,6 +77,23 @@ def test_exponent_shift_kat(zest_gpu, oracle):
     assert tiles.shape[0] > 0
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 200, 520), (300, 1000, 1024), (129, 333, 264)])
+def test_general_blocks_among_zero_blocks(zest_gpu, oracle, M, N, K):
+    """Weights of zero blocks with a few blocks of exponent bytes on both sides of 133 (the fast expansion's last):
+    the expansion leaves zero blocks alone and redoes the others. Whole numbers, so the result is exact. The padding
+    rows and columns are zero blocks as well."""
+    g = np.random.default_rng(M + N)
+    w = g.integers(-100, 101, (N, K // 8, 8)).astype(np.float32)
+    w *= np.exp2(g.integers(0, 7, (N, K // 8, 1)).astype(np.float32))   # exponent bytes up to 139
+    w[g.random((N, K // 8)) < 0.97] = 0.0
+    w[N // 2] = 0.0
+    x = g.integers(-3, 4, (M, K)).astype(np.float32)
+    c, nf, _, wp = run_gemm(zest_gpu, x, 0, w.reshape(N, K).view(np.uint8), N)
+    want = x.astype(np.float64) @ decoded(zest_gpu, oracle, wp, N, K).astype(np.float64).T
+    assert np.abs(want).max() < 2.0 ** 24 and nf == 0
+    assert np.array_equal(c.astype(np.float64), want)
+
+
 @pytest.mark.parametrize("wtype,M,N,K", [
     (8, 1024, 2560, 2560),   # BASELINE config 1 (test-mul-mat shape), Q8_0
     (12, 600, 896, 1536),    # padded widths and a ragged batch (test-mul-mat.cpp:153-156)
