@@ -399,6 +399,13 @@ __device__ inline float2 * rope_table(float * sh, int half, float pos, const rop
     return cs;
 }
 
+// A pair rotated. Which product of each sum is rounded is written out, so
+// every kernel gives the same bits (left to the compiler, each contracts its
+// sums its own way).
+__device__ inline float2 rotated(float x0, float x1, float2 r) {
+    return make_float2(fmaf(x0, r.x, -(x1 * r.y)), fmaf(x0, r.y, x1 * r.x));
+}
+
 __global__ __launch_bounds__(256) void rope_kernel(const float * __restrict__ x, int64_t heads, int64_t d,
                                                    const int32_t * __restrict__ pos, int n_dims, int neox,
                                                    rope_angles g, float * __restrict__ y) {
@@ -413,9 +420,9 @@ __global__ __launch_bounds__(256) void rope_kernel(const float * __restrict__ x,
         float * dst = y + (t * heads + h) * d;
         const int64_t ic = neox ? p : 2 * p;
         const float2 r = cs[p];
-        const float x0 = src[ic], x1 = src[ic + off];
-        dst[ic] = x0 * r.x - x1 * r.y;
-        dst[ic + off] = x0 * r.y + x1 * r.x;
+        const float2 o = rotated(src[ic], src[ic + off], r);
+        dst[ic] = o.x;
+        dst[ic + off] = o.y;
     }
     const int64_t rest = d - n_dims;
     if (rest > 0)
@@ -467,16 +474,13 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const float * __restrict_
             float * dst = yt + at(k);
             const float2 * r = cs + k % per * (NEOX ? 4 : 2);
             if (NEOX) {
-                *reinterpret_cast<float4 *>(dst) =
-                    make_float4(a[i].x * r[0].x - b[i].x * r[0].y, a[i].y * r[1].x - b[i].y * r[1].y,
-                                a[i].z * r[2].x - b[i].z * r[2].y, a[i].w * r[3].x - b[i].w * r[3].y);
-                *reinterpret_cast<float4 *>(dst + half) =
-                    make_float4(a[i].x * r[0].y + b[i].x * r[0].x, a[i].y * r[1].y + b[i].y * r[1].x,
-                                a[i].z * r[2].y + b[i].z * r[2].x, a[i].w * r[3].y + b[i].w * r[3].x);
+                const float2 o[4] = {rotated(a[i].x, b[i].x, r[0]), rotated(a[i].y, b[i].y, r[1]),
+                                     rotated(a[i].z, b[i].z, r[2]), rotated(a[i].w, b[i].w, r[3])};
+                *reinterpret_cast<float4 *>(dst) = make_float4(o[0].x, o[1].x, o[2].x, o[3].x);
+                *reinterpret_cast<float4 *>(dst + half) = make_float4(o[0].y, o[1].y, o[2].y, o[3].y);
             } else {
-                *reinterpret_cast<float4 *>(dst) =
-                    make_float4(a[i].x * r[0].x - a[i].y * r[0].y, a[i].x * r[0].y + a[i].y * r[0].x,
-                                a[i].z * r[1].x - a[i].w * r[1].y, a[i].z * r[1].y + a[i].w * r[1].x);
+                const float2 o[2] = {rotated(a[i].x, a[i].y, r[0]), rotated(a[i].z, a[i].w, r[1])};
+                *reinterpret_cast<float4 *>(dst) = make_float4(o[0].x, o[0].y, o[1].x, o[1].y);
             }
         }
     }
