@@ -438,7 +438,10 @@ __global__ __launch_bounds__(256) void rope_kernel(const float * __restrict__ x,
 // (normal) are whole pieces. Each thread requests its first ROPE_AHEAD pieces before
 // the table is made, so their latency and the table's overlap; HBM bound
 // (4096 x 48 x 128 with YaRN 47.2 -> 33.2 us, 201 MB; 2048 x 32 x 128 NeoX
-// 13.5 -> 11.4 us; 4096 x 8 x 128 12.9 -> 10.6).
+// 13.5 -> 11.4 us; 4096 x 8 x 128 12.9 -> 10.6). A token of few pieces takes
+// as many waves as hold them, so more tokens' tables are made at once (30000 x
+// 1 x 64 with four waves a token 24.4 us, slower than the 22.6 of the kernel
+// above; now 12.8).
 constexpr int ROPE_AHEAD = 4;
 
 template <bool NEOX>
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const float * __restrict_
                                                        float * __restrict__ y) {
     extern __shared__ float rope_sh[];
     constexpr int A = NEOX ? ROPE_AHEAD / 2 : ROPE_AHEAD;  // pieces in flight: 64 bytes a thread either way
-    const int half = n_dims / 2, per = (NEOX ? half : n_dims) / 4, n = heads * per;
+    const int half = n_dims / 2, per = (NEOX ? half : n_dims) / 4, n = heads * per, nt = blockDim.x;
     const int64_t t = blockIdx.x;
     const float * xt = x + t * heads * d;
     float * yt = y + t * heads * d;
@@ -456,7 +459,7 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const float * __restrict_
     auto load = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < A; i++) {
-            const int k = k0 + 256 * i;
+            const int k = k0 + nt * i;
             if (k < n) {
                 a[i] = *reinterpret_cast<const float4 *>(xt + at(k));
                 if (NEOX) b[i] = *reinterpret_cast<const float4 *>(xt + at(k) + half);
@@ -465,11 +468,11 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const float * __restrict_
     };
     load(threadIdx.x);
     const float2 * cs = rope_table(rope_sh, half, (float) pos[t], g);
-    for (int k0 = threadIdx.x; k0 < n; k0 += 256 * A) {
+    for (int k0 = threadIdx.x; k0 < n; k0 += nt * A) {
         if (k0 != (int) threadIdx.x) load(k0);
 #pragma unroll
         for (int i = 0; i < A; i++) {
-            const int k = k0 + 256 * i;
+            const int k = k0 + nt * i;
             if (k >= n) continue;
             float * dst = yt + at(k);
             const float2 * r = cs + k % per * (NEOX ? 4 : 2);
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const float * __restrict_
         }
     }
     const int rest = (d - n_dims) / 4;
-    for (int k = threadIdx.x; k < heads * rest; k += 256) {
+    for (int k = threadIdx.x; k < heads * rest; k += nt) {
         const int o = k / rest * d + n_dims + k % rest * 4;
         *reinterpret_cast<float4 *>(yt + o) = *reinterpret_cast<const float4 *>(xt + o);
     }
@@ -620,11 +623,13 @@ int zest_rope(const float * x, int64_t T, int64_t heads, int64_t d, const int32_
     // whole 16-byte pieces of every head (a token's offsets then fit 32 bits)
     const bool vec = d % 4 == 0 && (mode == 2 ? half : n_dims) % 4 == 0 && aligned16(x) && aligned16(y) &&
                      heads <= (1 << 30) / d;
+    const int64_t pieces = heads * std::max<int64_t>(mode == 2 ? half : n_dims, d - n_dims) / 4;
+    const dim3 threads(pieces <= 64 ? 64 : pieces <= 128 ? 128 : 256);
     if (vec && mode == 2)
-        hipLaunchKernelGGL(rope_vec_kernel<true>, dim3((unsigned) T), dim3(256), lds, s, x, (int) heads, (int) d, pos,
+        hipLaunchKernelGGL(rope_vec_kernel<true>, dim3((unsigned) T), threads, lds, s, x, (int) heads, (int) d, pos,
                            n_dims, g, y);
     else if (vec)
-        hipLaunchKernelGGL(rope_vec_kernel<false>, dim3((unsigned) T), dim3(256), lds, s, x, (int) heads, (int) d, pos,
+        hipLaunchKernelGGL(rope_vec_kernel<false>, dim3((unsigned) T), threads, lds, s, x, (int) heads, (int) d, pos,
                            n_dims, g, y);
     else
         hipLaunchKernelGGL(rope_kernel, dim3((unsigned) T), dim3(256), lds, s, x, heads, d, pos, n_dims, mode == 2, g,

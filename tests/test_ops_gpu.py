@@ -260,10 +260,11 @@ def test_rms_norm_narrow_rows(zest_gpu, oracle, rows, d):
 
 
 @pytest.mark.parametrize("neox", [False, True])
-@pytest.mark.parametrize("T,heads,d,n_dims", [(1, 1, 4, 4), (3, 5, 64, 64), (2, 33, 128, 128), (5, 48, 128, 96), (2, 7, 80, 72), (3, 3, 20, 10), (2, 2, 12, 8)])
+@pytest.mark.parametrize("T,heads,d,n_dims", [(1, 1, 4, 4), (3, 5, 64, 64), (2, 33, 128, 128), (5, 48, 128, 96), (2, 7, 80, 72), (3, 3, 20, 10),
+                                              (2, 2, 12, 8), (700, 1, 64, 64), (9, 8, 64, 64), (4, 9, 256, 32)])
 def test_rope_pieces(zest_gpu, T, heads, d, n_dims, neox):
-    """Rows of whole 16-byte pieces against the same rows one float off alignment, which take the float-by-float
-    kernel: the same bits."""
+    """Rows of whole 16-byte pieces, of one wave's pieces a token to several rounds of a workgroup's, against the same
+    rows one float off alignment, which take the float-by-float kernel: the same bits."""
     import torch
     x = _dev(Rng(T + heads + d).normal(T * heads * d, 0, 1.5).reshape(T, heads, d))
     pos = torch.tensor([5000 + 300 * i for i in range(T)], dtype=torch.int32, device="cuda")
