@@ -22,17 +22,17 @@ __device__ inline void pack4_expanded(uint8_t * packed, int64_t R_pad, int64_t r
     uint32_t e = 0;
 #pragma unroll
     for (int q = 0; q < 4; q++) e = max(e, (__float_as_uint(v[q]) >> 23) & 0xffu);
-    e = max(e, (uint32_t) __shfl_xor((int) e, 1));
+    e = max(e, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) e, 0xb1, 0xf, 0xf, true));  // lanes 1, 0, 3, 2
     const int sh = 133 - (int) e;
     const float sc = zest::block_scale(e);
     uint32_t b[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const int32_t qi =
-            (int32_t) __builtin_amdgcn_fmed3f(__builtin_rintf(__builtin_ldexpf(v[q], sh)), -128.0f, 127.0f);
-        b[q] = __float_as_uint((float) qi * sc) >> 16;  // exact: at most 8 significant bits
+        const float qf = __builtin_amdgcn_fmed3f(__builtin_rintf(__builtin_ldexpf(v[q], sh)), -128.0f, 127.0f);
+        b[q] = __float_as_uint(__builtin_fmaf(qf, sc, 0.0f));  // exact: at most 8 significant bits; + 0 makes -0 0
     }
-    *reinterpret_cast<uint2 *>(packed + zest_xoffset(r, c, R_pad)) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+    *reinterpret_cast<uint2 *>(packed + zest_xoffset(r, c, R_pad)) = make_uint2(
+        __builtin_amdgcn_perm(b[1], b[0], 0x07060302u), __builtin_amdgcn_perm(b[3], b[2], 0x07060302u));
 }
 
 // Zeroes row r of an expanded operand (d_pad columns): a padding row past the
@@ -249,46 +249,69 @@ __global__ __launch_bounds__(256) void rms_norm_narrow_kernel(const float * __re
     }
 }
 
-// y = act(g) * u (REGLU as g > 0 ? g*u : 0). A workgroup takes 16 rows by 256
-// columns, thread t row t/16 and the 4 floats at columns 64i + 4(t%16): the 16
-// threads of a row read 256 contiguous bytes at a time, every load issued
-// before the first activation, and a wave's packed store fills whole 128-byte
-// lines (4 rows by 16 columns each). HBM bound; a thread of 16 consecutive
-// columns, whose 16-byte loads lie 64 bytes apart across the lanes, is bound
-// by the vector cache instead (SWIGLU 2048 x 9728 packed 36.1 -> 30.2 us, 6.6
-// TB/s, to fp32 46.0 -> 35.5; 2286 x 17408 packed 102 -> 77). With a packed
-// output the grid also covers its padding rows and columns, written as zeros.
-template <int KIND>
+// y = act(g) * u (REGLU as g > 0 ? g*u : 0). A piece is 16 rows by 64 columns,
+// thread t row t/16 and the 4 floats at column 4(t%16), so the 16 threads of a
+// row read 256 contiguous bytes and a wave's packed store fills whole 128-byte
+// lines (4 rows by 16 columns each). A workgroup takes PIECES pieces that
+// follow each other along the rows (a row's last piece is followed by the
+// next rows' first, so narrow and ragged widths leave no thread idle), every
+// load issued before the first activation. HBM bound; a thread of 16
+// consecutive columns, whose 16-byte loads lie 64 bytes apart across the
+// lanes, is bound by the vector cache instead (SWIGLU 2048 x 9728 packed 36.1
+// -> 28.4 us, 7.0 TB/s, to fp32 45.5 -> 34.6). Two pieces where the tensors
+// stay in the 256 MB last-level cache or the result is packed alone (GEGLU
+// 2048 x 2560 packed 10.7 us, with four 11.9, with 256 columns of 16 rows a
+// workgroup 12.3; SWIGLU 30000 x 320 packed 14.9, 15.9 and 18.5), four where
+// an fp32 result takes them past it (2286 x 17408 84.5 us, with two 88.7).
+// With a packed output the grid also covers its padding rows and columns,
+// written as zeros.
+template <int KIND, int PIECES>
 __global__ __launch_bounds__(256) void glu_kernel(const float * __restrict__ g, int64_t sg, const float * __restrict__ u,
                                                   int64_t su, int64_t rows, int64_t f, float * __restrict__ y,
-                                                  uint8_t * __restrict__ packed, int64_t R_pad, unsigned nbx, bool vec,
-                                                  bool vec_y) {
-    const int t = threadIdx.x;
-    const int64_t r = (int64_t) (blockIdx.x / nbx) * 16 + (t >> 4), c0 = (int64_t) (blockIdx.x % nbx) * 256 + (t & 15) * 4;
-    const int64_t c_end = packed ? zest_k_padded(f) : f;
-    const bool row_ok = r < rows;
-    float4 gv[4], uv[4];
+                                                  uint8_t * __restrict__ packed, int64_t R_pad, unsigned across,
+                                                  unsigned pieces, bool vec, bool vec_y) {
+    const int tr = threadIdx.x >> 4, tc = (threadIdx.x & 15) * 4;
+    const unsigned first = blockIdx.x * PIECES;
+    // piece i's first row and column (uniform)
+    int64_t r0[PIECES], c0[PIECES];
+    unsigned band = first / across, at = first % across;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t c = c0 + 64 * i;
+    for (int i = 0; i < PIECES; i++) {
+        r0[i] = (int64_t) band * 16;
+        c0[i] = (int64_t) at * 64;
+        if (++at == across) {
+            at = 0;
+            band++;
+        }
+    }
+    const float * gt = g + tr * sg + tc;
+    const float * ut = u + tr * su + tc;
+    float4 gv[PIECES], uv[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; i++) {
+        const int64_t c = c0[i] + tc;
+        const bool row_ok = r0[i] + tr < rows;
+        const float * gp = gt + (r0[i] * sg + c0[i]);
+        const float * up = ut + (r0[i] * su + c0[i]);
         if (row_ok && vec && c + 4 <= f) {
-            gv[i] = *reinterpret_cast<const float4 *>(g + r * sg + c);
-            uv[i] = *reinterpret_cast<const float4 *>(u + r * su + c);
+            gv[i] = *reinterpret_cast<const float4 *>(gp);
+            uv[i] = *reinterpret_cast<const float4 *>(up);
         } else {
             float a[4], b[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                a[q] = row_ok && c + q < f ? g[r * sg + c + q] : 0.0f;
-                b[q] = row_ok && c + q < f ? u[r * su + c + q] : 0.0f;
+                a[q] = row_ok && c + q < f ? gp[q] : 0.0f;
+                b[q] = row_ok && c + q < f ? up[q] : 0.0f;
             }
             gv[i] = make_float4(a[0], a[1], a[2], a[3]);
             uv[i] = make_float4(b[0], b[1], b[2], b[3]);
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t c = c0 + 64 * i;
-        if (c >= c_end) break;  // pair-uniform where it matters: a packed row is whole 64-column tiles
+    for (int i = 0; i < PIECES; i++) {
+        if (first + i >= pieces) break;
+        const int64_t r = r0[i] + tr, c = c0[i] + tc;
+        const bool row_ok = r < rows;
         const float a[4] = {gv[i].x, gv[i].y, gv[i].z, gv[i].w}, b[4] = {uv[i].x, uv[i].y, uv[i].z, uv[i].w};
         float o[4];
 #pragma unroll
@@ -302,7 +325,8 @@ __global__ __launch_bounds__(256) void glu_kernel(const float * __restrict__ g, 
                     if (c + q < f) y[r * f + c + q] = o[q];
             }
         }
-        if (packed && r < R_pad) pack4_expanded(packed, R_pad, r, c, o);
+        // a whole piece: a packed operand is whole 64-column tiles of whole 16-row groups
+        if (packed) pack4_expanded(packed, R_pad, r, c, o);
     }
 }
 
@@ -562,16 +586,17 @@ int zest_glu(int kind, const float * g, int64_t sg, const float * u, int64_t su,
     ZEST_REQUIRE(!packed || f % 8 == 0, "zest_glu: packing needs f %% 8 == 0");
     ZEST_REQUIRE(aligned16(packed), "zest_glu: packed must be 16-byte aligned");
     const int64_t R_pad = zest_rows_padded(rows), gr = packed ? R_pad : rows;
-    const int64_t nbx = (f + 255) / 256, blocks = (gr + 15) / 16 * nbx;
-    ZEST_REQUIRE(blocks < (1ll << 31), "zest_glu: %lld x %lld is too large", (long long) rows, (long long) f);
-    const dim3 grid((unsigned) blocks);
+    const int64_t across = (f + 63) / 64, pieces = (gr + 15) / 16 * across;
+    ZEST_REQUIRE(pieces < (1ll << 31), "zest_glu: %lld x %lld is too large", (long long) rows, (long long) f);
+    const bool four = y && 3.0 * sizeof(float) * (double) rows * (double) f > (double) (256 << 20);
+    const dim3 grid(blocks_for(pieces, four ? 4 : 2));
     const bool vec = sg % 4 == 0 && su % 4 == 0 && aligned16(g) && aligned16(u), vec_y = f % 4 == 0 && aligned16(y);
     hipStream_t s = zest::as_stream(stream);
     uint8_t * p = (uint8_t *) packed;
 #define ZEST_GLU(KIND)                                                                                                  \
     case KIND:                                                                                                          \
-        hipLaunchKernelGGL(glu_kernel<KIND>, grid, dim3(256), 0, s, g, sg, u, su, rows, f, y, p, R_pad, (unsigned) nbx, \
-                           vec, vec_y);                                                                                 \
+        hipLaunchKernelGGL((four ? glu_kernel<KIND, 4> : glu_kernel<KIND, 2>), grid, dim3(256), 0, s, g, sg, u, su,     \
+                           rows, f, y, p, R_pad, (unsigned) across, (unsigned) pieces, vec, vec_y);                     \
         break
     switch (kind) {
         ZEST_GLU(ZEST_GLU_SWIGLU);

@@ -54,9 +54,10 @@ def test_glu_split(zest_gpu, oracle, kind):
     assert nrmse(got, oracle.glu(kind, g, u)) <= EXACT
 
 
-@pytest.mark.parametrize("rows,f,stride,shift", [(1, 8, 8, 0), (15, 264, 264, 0), (17, 1000, 1003, 0), (33, 256, 260, 1), (257, 72, 80, 4)])
+@pytest.mark.parametrize("rows,f,stride,shift", [(1, 8, 8, 0), (15, 264, 264, 0), (17, 1000, 1003, 0), (33, 256, 260, 1), (257, 72, 80, 4),
+                                                (300, 8, 8, 0), (49, 320, 320, 0)])
 def test_glu_edges(zest_gpu, oracle, rows, f, stride, shift):
-    """Rows and columns around the workgroup's 16 x 256, strides and starts that are not whole 16-byte pieces: the fp32
+    """Rows and columns around the 16 x 64 pieces and a workgroup's run of them, strides and starts that are not whole 16-byte pieces: the fp32
     result against the oracle, its pack the packer's, padding rows and columns zero."""
     import torch
     g = Rng(71).normal(rows * f, 0, 1.5).reshape(rows, f)
@@ -77,6 +78,24 @@ def test_glu_edges(zest_gpu, oracle, rows, f, stride, shift):
     packed.view(torch.uint8).fill_(255)
     zest_gpu.glu(1, *views, f, y=None, packed=packed)
     assert torch.equal(packed.view(torch.uint8), want.view(torch.uint8))
+
+
+def test_fused_pack_of_special_values(zest_gpu):
+    """The pack written by the GLU is the packer's of its fp32 result also where that holds NaN, infinities, zeros of
+    either sign and subnormals."""
+    import torch
+    g = np.random.default_rng(5)
+    x = g.normal(0, 1.5, (70, 328)).astype(np.float32)
+    for v in (np.nan, np.inf, -np.inf, -0.0, 0.0, 1e-40, -3e-39, -1.5e-45, 1e-37, 3e38):
+        x.reshape(-1)[g.integers(0, x.size, 40)] = v
+    x[3] = g.normal(0, 1e-38, 328)
+    x[4] = -0.0
+    xt, u = _dev(x), torch.ones(70, 328, device="cuda")
+    packed = zest_gpu.empty_act(70, 328)
+    for kind in range(5):
+        y = zest_gpu.glu(kind, xt, u, 328, packed=packed)
+        want = zest_gpu.pack_act_x(y)
+        assert torch.equal(packed.view(torch.uint8), want.view(torch.uint8)), kind
 
 
 @pytest.mark.parametrize("swapped", [False, True])
