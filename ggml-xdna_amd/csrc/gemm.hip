@@ -1195,7 +1195,10 @@ int cu_count(int dev) {
 std::mutex g_sk_mu;
 std::map<std::pair<int, hipStream_t>, sk_space> g_sk_spaces;
 
-// A split-K workspace of at least these sizes, in `out`. Nothing can be
+// A split-K workspace of at least these sizes, in `out`. The caller holds
+// g_sk_mu until its launch is queued: until then another thread's launch on
+// the stream could outgrow the workspace and free it, as its wait for the
+// stream would not cover this launch. Nothing can be
 // allocated while the stream is being captured: there `out.partial` is null
 // where the stream's workspace is too small (the launch then runs unsplit).
 int sk_reserve(hipStream_t s, size_t partial_bytes, size_t n_counters, sk_space & out, const char * name) {
@@ -1204,7 +1207,6 @@ int sk_reserve(hipStream_t s, size_t partial_bytes, size_t n_counters, sk_space 
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (s && hipStreamIsCapturing(s, &capture) != hipSuccess)
         return zest::fail(ZEST_E_HIP, "%s: hipStreamIsCapturing failed", name);
-    std::lock_guard<std::mutex> lock(g_sk_mu);
     sk_space & sp = g_sk_spaces[{dev, s}];
     const bool fits = sp.partial_bytes >= partial_bytes && sp.n_counters >= n_counters;
     out.partial = nullptr;
@@ -1394,6 +1396,7 @@ int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const ch
     const int64_t grid = T * p.splits;
     if (grid >= (1ll << 31) || (p.splits > 1 && grid * C::BM * C::BN * 4 >= (1ll << 31)))
         return zest::fail(ZEST_E_ARG, "%s: %lld tiles is too many", name, (long long) T);
+    std::unique_lock<std::mutex> lock(g_sk_mu, std::defer_lock);  // while the stream's workspace is in use here
     if (p.splits > 1) {
         const size_t partial_bytes = (size_t) grid * C::BM * C::BN * 4, n_counters = (size_t) T * (C::NC / 64);
         sk_space sp;
@@ -1407,6 +1410,7 @@ int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const ch
             hipLaunchKernelGGL(clear_counters, dim3((unsigned) ((n_counters + 255) / 256)), dim3(256), 0, s,
                                sp.counters, (int) n_counters);
         } else {
+            lock.lock();
             const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
             if (st != ZEST_OK) return st;
             // under capture, on a stream that no such launch has run on yet

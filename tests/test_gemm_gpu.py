@@ -684,3 +684,43 @@ def test_split_k_under_capture(zest_gpu, oracle):
                 s.synchronize()
         del g
     assert z.lib().zest_release_stream(s.cuda_stream) == 0
+
+
+def test_two_threads_on_one_stream(zest_gpu):
+    """Split launches of two sizes from two threads on one stream that holds no workspace yet: whichever grows it, the
+    other's launch keeps the memory it was given, and both give the bits they give alone."""
+    import threading
+    import torch
+    z = zest_gpu
+    s = torch.cuda.Stream()
+    jobs = []
+    for M, N, K in [(64, 512, 16384), (1024, 512, 16384)]:
+        a = z.pack_act_x(_dev(wide_blocks(M, K, 5)))
+        w = z.convert_weight(0, _dev(wide_blocks(N, K, 6, 0.02).view(np.uint8)), N, K)
+        want = z.gemm(a, M, w, N, K)
+        jobs.append((M, N, K, a, w, want, [torch.empty_like(want) for _ in range(8)]))
+    torch.cuda.synchronize()
+    lib, errors = z.lib(), []
+
+    def call(job, gate):
+        M, N, K, a, w, _, outs = job
+        gate.wait()
+        for o in outs:
+            if lib.zest_gemm(a.data_ptr(), M, w.data_ptr(), N, K, o.data_ptr(), N, None, s.cuda_stream) != 0:
+                errors.append(lib.zest_last_error())
+
+    for _ in range(4):
+        gate = threading.Barrier(2)
+        threads = [threading.Thread(target=call, args=(j, gate)) for j in jobs]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        s.synchronize()
+        assert not errors
+        for job in jobs:
+            for o in job[6]:
+                assert torch.equal(o.view(torch.int32), job[5].view(torch.int32)), job[:3]
+                o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        assert lib.zest_release_stream(s.cuda_stream) == 0
