@@ -28,6 +28,7 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -1192,8 +1193,16 @@ int cu_count(int dev) {
 }
 
 // The split-K workspaces, by device and stream (until zest_release_stream).
+// A stream as the workspaces are kept by: hipStreamPerThread is one handle for
+// a stream of each thread, so there the thread is part of it.
+using sk_stream = std::pair<hipStream_t, std::thread::id>;
+
+sk_stream sk_stream_of(hipStream_t s) {
+    return {s, s == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id()};
+}
+
 std::mutex g_sk_mu;
-std::map<std::pair<int, hipStream_t>, sk_space> g_sk_spaces;
+std::map<std::pair<int, sk_stream>, sk_space> g_sk_spaces;
 
 // A split-K workspace of at least these sizes, in `out`. The caller holds
 // g_sk_mu until its launch is queued: until then another thread's launch on
@@ -1207,7 +1216,7 @@ int sk_reserve(hipStream_t s, size_t partial_bytes, size_t n_counters, sk_space 
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (s && hipStreamIsCapturing(s, &capture) != hipSuccess)
         return zest::fail(ZEST_E_HIP, "%s: hipStreamIsCapturing failed", name);
-    sk_space & sp = g_sk_spaces[{dev, s}];
+    sk_space & sp = g_sk_spaces[{dev, sk_stream_of(s)}];
     const bool fits = sp.partial_bytes >= partial_bytes && sp.n_counters >= n_counters;
     out.partial = nullptr;
     if (capture != hipStreamCaptureStatusNone) {
@@ -1702,7 +1711,7 @@ extern "C" int zest_release_stream(void * stream) {
     std::lock_guard<std::mutex> lock(g_sk_mu);
     bool synced = false;
     for (auto it = g_sk_spaces.begin(); it != g_sk_spaces.end();) {
-        if (it->first.second != s) {
+        if (it->first.second != sk_stream_of(s)) {
             ++it;
             continue;
         }

@@ -168,7 +168,9 @@ ZEST_API int zest_gemm_group(const void *a, int64_t M, int64_t K, int n, const v
  * a stream that GEMMs ran on: the library cannot see a stream go, and a
  * process that makes and destroys streams would otherwise keep one workspace
  * per stream it ever used. A later GEMM on the stream allocates a new one;
- * a stream that holds none is left as it is. It has no counterpart in the
+ * a stream that holds none is left as it is. hipStreamPerThread is each
+ * thread's own stream, with a workspace of its own: a thread that ran GEMMs
+ * on it calls this before it ends. It has no counterpart in the
  * reference, whose NPU buffers live with its context. */
 ZEST_API int zest_release_stream(void *stream);
 

@@ -724,3 +724,39 @@ def test_two_threads_on_one_stream(zest_gpu):
                 o.fill_(float("nan"))
         torch.cuda.synchronize()
         assert lib.zest_release_stream(s.cuda_stream) == 0
+
+
+def test_per_thread_default_streams(zest_gpu):
+    """hipStreamPerThread is one handle for a stream of each thread: split launches on it from two threads, which may
+    overlap, have a workspace each and give the bits they give alone."""
+    import threading
+    import torch
+    z = zest_gpu
+    M, N, K, per_thread = 64, 512, 16384, 2  # hipStreamPerThread
+    jobs = []
+    for seed in (5, 7):
+        a = z.pack_act_x(_dev(wide_blocks(M, K, seed)))
+        w = z.convert_weight(0, _dev(wide_blocks(N, K, seed + 1, 0.02).view(np.uint8)), N, K)
+        want = z.gemm(a, M, w, N, K)
+        jobs.append((a, w, want, [torch.full_like(want, float("nan")) for _ in range(16)]))
+    torch.cuda.synchronize()
+    lib, errors, gate = z.lib(), [], threading.Barrier(2)
+
+    def call(a, w, _, outs):
+        gate.wait()
+        for o in outs:
+            if lib.zest_gemm(a.data_ptr(), M, w.data_ptr(), N, K, o.data_ptr(), N, None, per_thread) != 0:
+                errors.append(lib.zest_last_error())
+        if lib.zest_release_stream(per_thread) != 0:
+            errors.append(lib.zest_last_error())
+
+    threads = [threading.Thread(target=call, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for _, _, want, outs in jobs:
+        for o in outs:
+            assert torch.equal(o.view(torch.int32), want.view(torch.int32))
