@@ -54,6 +54,7 @@ SIGNATURES = {
     "zest_gemm_group": (_c_i, [_c_p, _c_i64, _c_i64, _c_i, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     "zest_gemm_group_noalloc": (_c_i, [_c_p, _c_i64, _c_i64, _c_i, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     "zest_release_stream": (_c_i, [_c_p]),
+    "zest_gemm_plan": (_c_i, [_c_i, _c_i64, _c_i64, _c_i, _c_p, _c_i, _c_p]),
     "zest_convert_weight_gu": (_c_i, [_c_i, _c_p, _c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "zest_gemm_glu": (_c_i, [_c_i, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p]),
     "zest_rms_norm": (_c_i, [_c_p, _c_i64, _c_i64, _c_f, _c_p, _c_p, _c_p, _c_p]),
@@ -252,6 +253,20 @@ def gemm_group(a_packed, m: int, weights, ns, k: int, outs=None, nonfinite=None,
     check(getattr(lib(), name)(_ptr(a_packed), m, k, n, w, I64(*ns), c, I64(*[t.stride(0) for t in outs]),
                                _ptr(nonfinite), _stream()), name)
     return outs
+
+
+class _Plan(ctypes.Structure):
+    _fields_ = ([(f, ctypes.c_int32) for f in ("tile_rows", "tile_cols", "waves", "k_groups", "per_cu", "splits")] +
+                [(f, ctypes.c_int64) for f in ("tiles", "whole_tiles", "workspace")])
+
+
+def gemm_plan(m: int, ns, k: int, kind: int = -1, cus: int = 256) -> dict:
+    """The plan of a GEMM launch (zest_gemm_plan; no GPU needed). kind: -1 plain or group, -2 residual, a GLU kind
+    (ns then [2F])."""
+    out = _Plan()
+    check(lib().zest_gemm_plan(kind, m, k, len(ns), (ctypes.c_int64 * len(ns))(*ns), cus, ctypes.byref(out)),
+          "zest_gemm_plan")
+    return {f: getattr(out, f) for f, _ in _Plan._fields_}
 
 
 def convert_weight_gu(wtype: int, gate, up, f: int, k: int, out=None):

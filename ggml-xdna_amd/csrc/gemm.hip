@@ -1383,13 +1383,10 @@ double plan_us(const shape_rate & r, int64_t T, int nk, int64_t P, int S) {
     return S == 1 ? t : t + 0.75 * S + 2.0 * (double) U * r.bm * r.bn * 4 / 8e6;
 }
 
-// Plans and launches one GEMM (a group of weights, or the fused GLU). A
-// split-K plan takes its workspace from `fixed` when given (no allocation:
-// a plan that does not fit is rejected, and the counters it uses are cleared
-// first), else from the per-stream workspace.
+// Launches one GEMM (a group of weights, or the fused GLU) as tiles of C in
+// `splits` K splits, whose partial sums go through the workspace `sp`.
 template <class C, int EPI>
-int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const char * name,
-           const sk_space * fixed = nullptr) {
+int launch(gemm_params p, const int64_t * N, int splits, const sk_space & sp, hipStream_t s, const char * name) {
     p.mt = (int) ((p.M + C::BM - 1) / C::BM);
     int nt = 0;
     for (int i = 0; i < p.nw; i++) {
@@ -1405,29 +1402,8 @@ int launch(gemm_params p, const int64_t * N, int splits, hipStream_t s, const ch
     const int64_t grid = T * p.splits;
     if (grid >= (1ll << 31) || (p.splits > 1 && grid * C::BM * C::BN * 4 >= (1ll << 31)))
         return zest::fail(ZEST_E_ARG, "%s: %lld tiles is too many", name, (long long) T);
-    std::unique_lock<std::mutex> lock(g_sk_mu, std::defer_lock);  // while the stream's workspace is in use here
-    if (p.splits > 1) {
-        const size_t partial_bytes = (size_t) grid * C::BM * C::BN * 4, n_counters = (size_t) T * (C::NC / 64);
-        sk_space sp;
-        if (fixed) {
-            if (partial_bytes > fixed->partial_bytes || n_counters > fixed->n_counters)
-                return zest::fail(ZEST_E_ARG,
-                                  "%s: this shape's split-K plan needs %zu bytes of partial sums and %zu counters; "
-                                  "the static workspace holds %zu bytes and %zu counters",
-                                  name, partial_bytes, n_counters, fixed->partial_bytes, fixed->n_counters);
-            sp = *fixed;
-            hipLaunchKernelGGL(clear_counters, dim3((unsigned) ((n_counters + 255) / 256)), dim3(256), 0, s,
-                               sp.counters, (int) n_counters);
-        } else {
-            lock.lock();
-            const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
-            if (st != ZEST_OK) return st;
-            // under capture, on a stream that no such launch has run on yet
-            if (!sp.partial) return launch<C, EPI>(p, N, 1, s, name);
-        }
-        p.partial = sp.partial;
-        p.counters = sp.counters;
-    }
+    p.partial = sp.partial;
+    p.counters = sp.counters;
 #if ZEST_GEMM_PERSIST
     // more than one round: persistent workgroups, one a CU (not for the
     // residual epilogue, whose persistent form does not fit the registers)
@@ -1492,31 +1468,37 @@ int launch_mixed(gemm_params p, const int64_t * N, int64_t nbig, hipStream_t s, 
     return zest::check_launch(name);
 }
 
-// The plan of a plain (or residual) launch: its tile shape and K splits.
-struct plain_plan {
+// A launch's plan: its tile shape, K splits and, for a mixed launch, how many
+// of its 256x128 tiles run whole.
+struct gemm_plan {
     int kind = SHAPE_BIG;
     int splits = 1;
-    int64_t nbig = 0;  // mixed: the whole tiles
+    int64_t nbig = 0;
     double us = 1e300;
 };
 
-// The cheapest plan by the cost model: a tile shape with its K splits, or a
-// mixed launch. A launch whose whole tiles fill every CU is not split, a split
+// The split-K workspace of T tiles of shape k in S splits.
+size_t partial_bytes_of(int k, int64_t T, int S) { return (size_t) (T * S) * RATES[k].bm * RATES[k].bn * 4; }
+size_t counters_of(int k, int64_t T) { return (size_t) T * RATES[k].waves; }
+
+// The cheapest plan of a plain (or residual) launch by the cost model: a tile
+// shape with its K splits, or a mixed launch. A launch whose whole tiles fill
+// every CU is not split, a split
 // keeps at least three K-steps a K-group, and the partial sums of K up to 32768
 // fit the static workspace of zest_gemm_group_noalloc, which runs the same
 // plan (only a longer K is worth more: 2048 x 2816 x 65536 in four splits).
-plain_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P) {
-    plain_plan best;
+gemm_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P, int max_splits) {
+    gemm_plan best;
     bool whole = true;  // every weight whole 160-row tiles
     for (int i = 0; i < p.nw; i++) whole &= N[i] % cfg_o::BN == 0;
     for (int k = 0; k < SHAPES; k++) {
         const shape_rate & r = RATES[k];
         if (k == SHAPE_O && !whole) continue;
         const int64_t T = tiles_of(p, N, r.bm, r.bn), slots = P * r.per_cu;
-        for (int S = 1; S <= ZEST_GEMM_MAX_SPLIT; S++) {
+        for (int S = 1; S <= max_splits; S++) {
             if (S > 1 && (T >= slots || T * S > 4 * slots || p.nk < 3 * S * r.kg)) break;
             if (S > 1 && (p.nk <= 512 || whole) &&
-                (T * S * r.bm * r.bn * 4 > (int64_t) ZEST_NOALLOC_PARTIAL_BYTES || T * r.waves > ZEST_NOALLOC_COUNTERS))
+                (partial_bytes_of(k, T, S) > ZEST_NOALLOC_PARTIAL_BYTES || counters_of(k, T) > ZEST_NOALLOC_COUNTERS))
                 break;
             if (r.kg > 1 && (p.nk % (S * r.kg) || p.nk < 2 * S * r.kg)) continue;
             const double us = plan_us(r, T, p.nk, P, S);
@@ -1535,57 +1517,82 @@ plain_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P) {
     return best;
 }
 
-// Plans and launches a GEMM; `fixed` as for launch(). A fused GLU launch
-// splits K as the plain launch of its 2F columns would, in as many K-groups
-// (so its gate and up sums are that launch's, bit for bit: a sum depends on
-// the K-steps' partition and order, not on the tile shape), and takes the
-// cheapest of its tile shapes for that partition.
+// The columns that a fused GLU's tiles cover: the output operand's K padding
+// too, the columns of 2F rounded up to 128 rows of the gate/up pair, whose
+// rows past 2F are zero blocks, so the h columns past F store the packer's
+// zeros (with 64-column tiles and F % 64 == 32 the last tile would end at F).
+int64_t glu_columns(int64_t N) { return (N + 127) / 128 * 128; }
+
+// The plan of a launch with epilogue `epi`. A fused GLU launch splits K as the
+// plain launch of its 2F columns would, in as many K-groups (so its gate and
+// up sums are that launch's, bit for bit: a sum depends on the K-steps'
+// partition and order, not on the tile shape), and takes the cheapest of its
+// tile shapes for that partition.
+gemm_plan plan_of(int epi, const gemm_params & p, const int64_t * N, int64_t P, int max_splits) {
+    const gemm_plan plain = plan_plain(p, N, P, max_splits);
+    if (epi < 0) return plain;
+    const int64_t Nt = glu_columns(N[0]);
+    const int kg = plain.kind == SHAPE_MIXED ? 1 : RATES[plain.kind].kg;
+    gemm_plan best;
+    for (const int k : {SHAPE_GLU, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2}) {
+        const shape_rate & r = RATES[k];
+        if (r.kg != kg) continue;
+        const double us = plan_us(r, tiles_of(p, &Nt, r.bm, r.bn), p.nk, P, plain.splits);
+        if (us < best.us) best = {k, plain.splits, 0, us};
+    }
+    return best;
+}
+
+// Plans and launches a GEMM. A split-K plan takes its workspace from `fixed`
+// when given (no allocation: a plan that does not fit is rejected, and the
+// counters it uses are cleared first), else from the stream's, in use here
+// until the launch is queued. Under capture on a stream whose workspace is
+// too small it runs unsplit.
 template <int EPI>
-int launch_any(gemm_params p, const int64_t * N, hipStream_t s, const char * name,
+int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const char * name,
                const sk_space * fixed = nullptr) {
     int dev = 0;
     (void) hipGetDevice(&dev);
-    const int64_t P = cu_count(dev);
-    const plain_plan pp = plan_plain(p, N, P);
-    const int S = pp.splits;
-    if constexpr (EPI >= 0) {
-        // The tiles cover the output operand's K padding too: the columns of
-        // 2F rounded up to 128 rows of the gate/up pair, whose rows past 2F
-        // are zero blocks, so the h columns past F store the packer's zeros
-        // (with 64-column tiles and F % 64 == 32 the last tile would end at F).
-        const int64_t Nt = (N[0] + 127) / 128 * 128;
-        const int kg = pp.kind == SHAPE_MIXED ? 1 : RATES[pp.kind].kg;
-        int kind = SHAPES;
-        double least = 1e300;
-        for (const int k : {SHAPE_GLU, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2}) {
-            if (RATES[k].kg != kg) continue;
-            const double us = plan_us(RATES[k], tiles_of(p, &Nt, RATES[k].bm, RATES[k].bn), p.nk, P, S);
-            if (us < least) {
-                kind = k;
-                least = us;
-            }
-        }
-        switch (kind) {
-            case SHAPE_SMALL: return launch<cfg_small, EPI>(p, &Nt, S, s, name, fixed);
-            case SHAPE_MID: return launch<cfg_mid, EPI>(p, &Nt, S, s, name, fixed);
-            case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, &Nt, S, s, name, fixed);
-            case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, &Nt, S, s, name, fixed);
-            case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, &Nt, S, s, name, fixed);
-            default: return launch<cfg_glu, EPI>(p, &Nt, S, s, name, fixed);
-        }
-    } else {
-        switch (pp.kind) {
-            case SHAPE_GLU: return launch<cfg_glu, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_O: return launch<cfg_o, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_SMALL: return launch<cfg_small, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_MID: return launch<cfg_mid, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, N, S, s, name, fixed);
-            case SHAPE_MIXED: return launch_mixed<cfg_glu, cfg_half8, EPI>(p, N, pp.nbig, s, name);
-            default: return launch<cfg_big, EPI>(p, N, S, s, name, fixed);
+    const int64_t P = cu_count(dev), Nt = glu_columns(N[0]);
+    const int64_t * cols = EPI >= 0 ? &Nt : N;
+    gemm_plan pp = plan_of(EPI, p, N, P, ZEST_GEMM_MAX_SPLIT);
+    std::unique_lock<std::mutex> lock(g_sk_mu, std::defer_lock);
+    sk_space sp;
+    if (pp.splits > 1) {
+        const int64_t T = tiles_of(p, cols, RATES[pp.kind].bm, RATES[pp.kind].bn);
+        const size_t partial_bytes = partial_bytes_of(pp.kind, T, pp.splits), n_counters = counters_of(pp.kind, T);
+        if (fixed) {
+            if (partial_bytes > fixed->partial_bytes || n_counters > fixed->n_counters)
+                return zest::fail(ZEST_E_ARG,
+                                  "%s: this shape's split-K plan needs %zu bytes of partial sums and %zu counters; "
+                                  "the static workspace holds %zu bytes and %zu counters",
+                                  name, partial_bytes, n_counters, fixed->partial_bytes, fixed->n_counters);
+            sp = *fixed;
+            hipLaunchKernelGGL(clear_counters, dim3((unsigned) ((n_counters + 255) / 256)), dim3(256), 0, s,
+                               sp.counters, (int) n_counters);
+        } else {
+            lock.lock();
+            const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
+            if (st != ZEST_OK) return st;
+            if (!sp.partial) pp.splits = 1;
         }
     }
+    const int S = pp.splits;
+    switch (pp.kind) {
+        case SHAPE_GLU: return launch<cfg_glu, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_SMALL: return launch<cfg_small, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_MID: return launch<cfg_mid, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, cols, S, sp, s, name);
+        default: break;
+    }
+    if constexpr (EPI < 0) {
+        if (pp.kind == SHAPE_BIG) return launch<cfg_big, EPI>(p, N, S, sp, s, name);
+        if (pp.kind == SHAPE_O) return launch<cfg_o, EPI>(p, N, S, sp, s, name);
+        if (pp.kind == SHAPE_MIXED) return launch_mixed<cfg_glu, cfg_half8, EPI>(p, N, pp.nbig, s, name);
+    }
+    return zest::fail(ZEST_E_ARG, "%s: no plan", name);
 }
 
 // The parts of a launch's parameters common to every kind.
@@ -1704,6 +1711,25 @@ extern "C" int zest_gemm_group_noalloc(const void * a, int64_t M, int64_t K, int
                                        const int64_t * N, float * const * c, const int64_t * ldc,
                                        uint32_t * nonfinite, void * stream) {
     return gemm_group(a, M, K, n, w, N, c, ldc, nonfinite, stream, "zest_gemm_group_noalloc", true);
+}
+
+extern "C" int zest_gemm_plan(int kind, int64_t M, int64_t K, int n, const int64_t * N, int cus, zest_plan * out) {
+    ZEST_REQUIRE(N && out, "zest_gemm_plan: null pointer");
+    ZEST_REQUIRE(kind >= ZEST_PLAN_RESIDUAL && kind <= ZEST_GLU_GEGLU_QUICK, "zest_gemm_plan: kind %d", kind);
+    ZEST_REQUIRE(n >= 1 && n <= (kind == ZEST_PLAN_PLAIN ? ZEST_GEMM_MAX_GROUP : 1), "zest_gemm_plan: %d weights", n);
+    ZEST_REQUIRE(M > 0 && K > 0 && K % 8 == 0 && cus > 0, "zest_gemm_plan: M=%lld K=%lld cus=%d", (long long) M,
+                 (long long) K, cus);
+    for (int i = 0; i < n; i++) ZEST_REQUIRE(N[i] > 0, "zest_gemm_plan: N[%d]=%lld", i, (long long) N[i]);
+    static_assert(ZEST_PLAN_PLAIN == EPI_PLAIN && ZEST_PLAN_RESIDUAL == EPI_RESIDUAL, "a plan's kinds are the epilogues");
+    gemm_params p = base_params(nullptr, M, K, nullptr);
+    p.nw = n;
+    const gemm_plan plan = plan_of(kind, p, N, cus, ZEST_GEMM_MAX_SPLIT);
+    const bool mixed = plan.kind == SHAPE_MIXED;
+    const shape_rate & t = RATES[mixed ? (int) SHAPE_GLU : plan.kind];
+    const int64_t Nt = glu_columns(N[0]), T = tiles_of(p, kind >= 0 ? &Nt : N, t.bm, t.bn);
+    *out = {t.bm, t.bn, t.waves, t.kg, t.per_cu, plan.splits, T, mixed ? plan.nbig : T,
+            plan.splits > 1 ? (int64_t) partial_bytes_of(plan.kind, T, plan.splits) : 0};
+    return ZEST_OK;
 }
 
 extern "C" int zest_release_stream(void * stream) {

@@ -163,6 +163,26 @@ ZEST_API int zest_gemm_residual(const void *a, int64_t M, const void *w, int64_t
 ZEST_API int zest_gemm_group(const void *a, int64_t M, int64_t K, int n, const void *const *w, const int64_t *N,
                              float *const *c, const int64_t *ldc, uint32_t *nonfinite, void *stream);
 
+/* The plan that a GEMM launch of these sizes takes on a GPU of `cus` compute
+ * units: host arithmetic only, no GPU needed (tests and diagnostics read it;
+ * it has no counterpart in the reference). kind: ZEST_PLAN_PLAIN for
+ * zest_gemm and zest_gemm_group, ZEST_PLAN_RESIDUAL for zest_gemm_residual, a
+ * GLU kind for zest_gemm_glu (n = 1, N[0] = 2F). An output that runs as bands
+ * of rows has a plan for each band's M. */
+#define ZEST_PLAN_PLAIN (-1)
+#define ZEST_PLAN_RESIDUAL (-2)
+typedef struct {
+    int32_t tile_rows, tile_cols; /* a tile of the output */
+    int32_t waves;                /* consumer waves of a K-group */
+    int32_t k_groups;             /* K-groups of a workgroup */
+    int32_t per_cu;               /* workgroups a CU */
+    int32_t splits;               /* K splits among workgroups */
+    int64_t tiles;                /* tiles of that shape */
+    int64_t whole_tiles;          /* of them, run whole (a mixed launch runs the others as halves) */
+    int64_t workspace;            /* bytes of partial sums, 0 unsplit */
+} zest_plan;
+ZEST_API int zest_gemm_plan(int kind, int64_t M, int64_t K, int n, const int64_t *N, int cus, zest_plan *out);
+
 /* Frees the split-K workspace the library holds for `stream` (on every
  * device), after the launches queued on it finish. Call it before destroying
  * a stream that GEMMs ran on: the library cannot see a stream go, and a

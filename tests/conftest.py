@@ -18,6 +18,15 @@ def oracle():
 
 
 @pytest.fixture(scope="session")
+def zest():
+    """The package with its library loaded, for what needs no GPU."""
+    from helpers import load_pkg
+    z = load_pkg()
+    z.lib()
+    return z
+
+
+@pytest.fixture(scope="session")
 def zest_gpu():
     """The package with its library loaded and device 0 initialised; the GPU
     tests must run through it (no fallback)."""
