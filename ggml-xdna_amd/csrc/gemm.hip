@@ -1547,7 +1547,7 @@ gemm_plan plan_of(int epi, const gemm_params & p, const int64_t * N, int64_t P, 
 // when given (no allocation: a plan that does not fit is rejected, and the
 // counters it uses are cleared first), else from the stream's, in use here
 // until the launch is queued. Under capture on a stream whose workspace is
-// too small it runs unsplit.
+// too small it is the best unsplit plan instead.
 template <int EPI>
 int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const char * name,
                const sk_space * fixed = nullptr) {
@@ -1574,7 +1574,7 @@ int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const ch
             lock.lock();
             const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
             if (st != ZEST_OK) return st;
-            if (!sp.partial) pp.splits = 1;
+            if (!sp.partial) pp = plan_of(EPI, p, N, P, 1);
         }
     }
     const int S = pp.splits;

@@ -151,12 +151,18 @@ ZEST_API int zest_gemm_residual(const void *a, int64_t M, const void *w, int64_t
  * use (and grows, synchronizing the stream; zest_release_stream frees it):
  * calls that share a stream run in order and never share it concurrently.
  * Under stream capture nothing is allocated: a launch whose stream does not
- * hold a large enough workspace yet runs unsplit, and one that a graph was
- * captured with is kept until zest_release_stream, also when a later call
- * outgrows it (a replay uses it, so replays must not overlap calls on the
- * stream it was captured on). A launch of at most one small
- * tile a CU may instead split each tile's K between two groups of waves in
- * one workgroup (K-groups), whose sums meet in LDS, also in a fixed order.
+ * hold a large enough workspace yet takes the best unsplit plan, whose sums
+ * are rounded in another order. What this header says of calls that give each
+ * other's bits (residual and plain, GLU and plain, this call and
+ * zest_gemm_group_noalloc) holds for captured calls only where the same calls
+ * ran on the stream before the capture. A workspace that a graph was captured
+ * with is kept until zest_release_stream, also when a later call outgrows it:
+ * replays use it, so they must overlap neither calls on the stream that was
+ * captured nor replays of other graphs captured on it, on whatever streams
+ * they run (torch captures on one stream of its own unless given another).
+ * A launch of small tiles may also split each tile's K between two groups of
+ * waves in one workgroup (K-groups), whose sums meet in LDS, also in a fixed
+ * order.
  * The same holds for zest_gemm and zest_gemm_glu, which run through the
  * same launch. */
 #define ZEST_GEMM_MAX_GROUP 4

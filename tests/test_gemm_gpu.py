@@ -760,3 +760,57 @@ def test_per_thread_default_streams(zest_gpu):
     for _, _, want, outs in jobs:
         for o in outs:
             assert torch.equal(o.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("form", ["residual", "glu"])
+def test_split_k_forms_under_capture(zest_gpu, form):
+    """The residual and the fused GLU form of a split plan captured on a stream that ran it before: each replay gives
+    the eager call's bits, which are the plain call's plus the add, and the unfused chain's. Captured on a stream that
+    has no workspace the unsplit plan runs: the replays agree with each other and are close to the eager call."""
+    import torch
+    z = zest_gpu
+    M, N, K = 64, 512, 16384
+    assert z.gemm_plan(M, [N], K)["splits"] > 1
+    F = N // 2
+    a = z.pack_act_x(_dev(wide_blocks(M, K, 5)))
+    out = torch.empty((M, N if form == "residual" else F), device="cuda")
+    if form == "residual":
+        w = z.convert_weight(0, _dev(wide_blocks(N, K, 6, 0.02).view(np.uint8)), N, K)
+        res = torch.randn((M, N), device="cuda")
+        call = lambda: z.gemm_residual(a, M, w, N, K, res, out=out)
+        want = z.add(z.gemm(a, M, w, N, K), res)
+    else:
+        gate, up = (_dev(wide_blocks(F, K, i, 0.02).view(np.uint8)) for i in (6, 7))
+        w = z.convert_weight_gu(0, gate, up, F, K)
+        call = lambda: z.gemm_glu(0, a, M, w, F, K, xout=None, h=out)
+        c = z.gemm(a, M, w, N, K).view(M, F // 32, 2, 32)
+        want = z.glu(0, c[:, :, 0, :].reshape(M, F).contiguous(), c[:, :, 1, :].reshape(M, F).contiguous(), F)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for warm in (False, True):
+        if warm:
+            with torch.cuda.stream(s):
+                call()
+            s.synchronize()
+            assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            call()
+        torch.cuda.synchronize()
+        first = None
+        for rep in range(3):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            first = out.clone() if first is None else first
+            assert torch.equal(out.view(torch.int32), (want if warm else first).view(torch.int32)), (warm, rep)
+            with torch.cuda.stream(s):
+                z.gemm_group(a, M, [w], [N], K)
+            s.synchronize()
+        # sums of K products in another order: each within 2 K 2^-24 of sum |a b|, here of its largest
+        assert float((first - want).norm() / want.norm()) <= 1e-4
+        del g
+        if not warm:
+            assert z.lib().zest_release_stream(s.cuda_stream) == 0
+    assert z.lib().zest_release_stream(s.cuda_stream) == 0
