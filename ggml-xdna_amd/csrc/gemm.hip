@@ -25,6 +25,7 @@
 // steps while it finishes the current one (gemm_kernel_tiles; mixed launches:
 // gemm_kernel_mixed_tiles).
 #include <algorithm>
+#include <cmath>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -1122,7 +1123,9 @@ using cfg_o = gemm_cfg<128, 160, 4, 384, 1, 1, 128>;
 // thread, 0.36 of them the producers alone and 0.24 the consumers alone. So
 // they have producers of one unit a thread, two waves on each SIMD whose
 // steps overlap, and 8 consumers where 4 would leave a SIMD's other wave to
-// wait for (128x128: 0.36 us; 1024 x 2560 x 2560 21.4 -> 20.0 us).
+// wait for. 128x128 so: 0.36 us a step; the fastest for wide weights over up to
+// 128 rows (98 x (8704 + 8704) x 2816 behind its norm 19.4 us, as 128x64 tiles
+// 22.1; fused, 108 x 18432 x 3584, 26.7 and 30.4).
 using cfg_small = gemm_cfg<128, 128, 4, 512, 1, 2, 512>;
 // 128x64 tiles, two workgroups a CU (2048 x 1024 x 4096 31.6 -> 25.2 us, where
 // 64x64 tiles were the best before), and as two K-groups, one workgroup a CU,
@@ -1137,6 +1140,13 @@ using cfg_mid2 = gemm_cfg<128, 64, 4, 256, 1, 1, 256, 2>;
 // two K splits; 48 x 19456 x 2560, 304 tiles, 20.9 with the first, 18.5 with the second).
 using cfg_tiny2 = gemm_cfg<64, 64, 2, 256, 1, 1, 256, 2>;
 using cfg_tiny2x2 = gemm_cfg<64, 64, 2, 128, 2, 1, 0, 2>;
+// 64x64 tiles of one K-group: four waves of 96 registers and a 24 KB ring, so
+// up to five workgroups a CU, for wide weights over few rows, where they are
+// what keeps enough of W in flight (32 x (17408 + 17408) x 5120: 39.4 us, 5.1
+// TB/s, against 44.5 as K-groups; 32 x 5945 x 6688 16.2 in five K splits against
+// 20.7; 32 x 41572 x 1024 12.2 against 16.1), and for short K over many tiles (1833 x
+// 2304 x 384 with the residual 11.0 against 12.3).
+using cfg_tiny = gemm_cfg<64, 64, 2, 128, 5>;
 // Mixed launches run their whole tiles as cfg_glu's (two consumers per SIMD)
 // and the halves as 128x128 tiles of 8 consumer waves of 32x64 (4 row blocks
 // x 2 column blocks) and 4 producers, the same threads (the q/k/v group at
@@ -1316,73 +1326,6 @@ int set_lds_mixed(const char * name) {
     return ZEST_OK;
 }
 
-// Tiles of a launch for one tile shape.
-int64_t tiles_of(const gemm_params & p, const int64_t * N, int BM, int BN) {
-    int64_t nt = 0;
-    for (int i = 0; i < p.nw; i++) nt += (N[i] + BN - 1) / BN;
-    return ((p.M + BM - 1) / BM) * nt;
-}
-
-// The launch cost model, in microseconds. U = T * S units (T tiles in S K
-// splits) on P CUs of `per_cu` workgroups each take whole rounds of P * per_cu
-// units and a last, partly filled one. A unit runs its K-steps (nk / (S * kg))
-// and `prologue` more (the pipeline's fill and the epilogue); a step takes
-// `step` with the GPU nearly idle and `full` times that in a whole round (the
-// clock falls under the power limit and the L2s fill up). In between it rises
-// with the square of the share of CUs at work; where two workgroups fit a CU, to
-// 1 + `load` with one on each, then, once any CU has two, on a line from `pair`
-// to `full` (128x64 tiles, a step's time over one workgroup's: 1.6 with 1.1 a CU,
-// 2.0 with 2). A split launch pays for its partial sums: each unit writes its tile
-// and the last ones read them back, 2 * U * BM*BN*4 bytes at about 8 TB/s, and
-// 0.75 us a split for their round trips. The numbers are a fit of the choice
-// itself to some 6000 launches timed one plan after another (18 weight shapes of
-// hidden sizes 1024 to 5120, 48 to 3000 rows), then to 957 launches with all
-// their plans over all widths and 32 to 4096 rows, the fused and the residual
-// ones among them: over these the choice takes 0.4% longer than the best plan
-// measured for each, where the first fit, which had a square of the share for
-// two workgroups a CU as well, took 1.0% (773 x 2816 x 11008 with 1.2 such
-// workgroups a CU 79 us, its best plan 63).
-struct shape_rate {
-    int bm, bn, kg, per_cu, waves;  // waves: consumer waves, a counter each in a split launch
-    double fixed, prologue, step, load, pair, full;
-};
-
-template <class C>
-constexpr shape_rate rate_of(double fixed, double prologue, double step, double load) {
-    static_assert(C::MINB == 1, "one workgroup a CU");
-    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load, 0.0, 1 + load};
-}
-
-template <class C>
-constexpr shape_rate rate_of(double fixed, double prologue, double step, double load, double pair, double full) {
-    static_assert(C::MINB == 2, "two workgroups a CU");
-    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64, fixed, prologue, step, load, pair, full};
-}
-
-enum shape_kind { SHAPE_BIG, SHAPE_GLU, SHAPE_O, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2, SHAPES, SHAPE_MIXED };
-
-constexpr shape_rate RATES[SHAPES] = {
-    rate_of<cfg_big>(8.45, 4.53, 0.455, 0.470),    rate_of<cfg_glu>(5.34, 4.18, 0.455, 0.553),
-    rate_of<cfg_o>(3.87, 7.38, 0.353, 0.475),      rate_of<cfg_small>(2.68, 4.59, 0.391, 0.456),
-    rate_of<cfg_mid>(2.54, 7.26, 0.222, 0.294, 1.642, 1.929), rate_of<cfg_mid2>(2.72, 4.47, 0.350, 0.343),
-    rate_of<cfg_tiny2>(2.90, 3.56, 0.2795, 0.233), rate_of<cfg_tiny2x2>(2.64, 5.94, 0.305, 0.216, 1.675, 1.817),
-};
-
-// U units of `steps` K-steps, in rounds of `slots`
-double rounds_us(const shape_rate & r, int64_t U, double steps, int64_t slots) {
-    const double f = (double) (U % slots) / (double) slots, step = (steps + r.prologue) * r.step;
-    double last = 0.0;  // the last, partly filled round
-    if (U % slots && r.per_cu == 1) last = 1 + r.load * f * f;
-    else if (U % slots) last = 2 * f <= 1 ? 1 + r.load * 4 * f * f : r.pair + (r.full - r.pair) * (2 * f - 1);
-    return step * ((double) (U / slots) * r.full + last);
-}
-
-double plan_us(const shape_rate & r, int64_t T, int nk, int64_t P, int S) {
-    const int64_t U = T * S;
-    const double t = r.fixed + rounds_us(r, U, (double) nk / (S * r.kg), P * r.per_cu);
-    return S == 1 ? t : t + 0.75 * S + 2.0 * (double) U * r.bm * r.bn * 4 / 8e6;
-}
-
 // Launches one GEMM (a group of weights, or the fused GLU) as tiles of C in
 // `splits` K splits, whose partial sums go through the workspace `sp`.
 template <class C, int EPI>
@@ -1468,6 +1411,187 @@ int launch_mixed(gemm_params p, const int64_t * N, int64_t nbig, hipStream_t s, 
     return zest::check_launch(name);
 }
 
+enum shape_kind {
+    SHAPE_BIG, SHAPE_GLU, SHAPE_O, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2, SHAPE_TINY, SHAPES,
+    SHAPE_MIXED
+};
+
+struct tile_shape {
+    int bm, bn, kg, per_cu, waves;  // waves: consumer waves, a counter each in a split launch
+};
+
+template <class C>
+constexpr tile_shape shape_of() {
+    return {C::BM, C::BN, C::KG, C::MINB, C::NC / 64};
+}
+
+constexpr tile_shape TILES[SHAPES] = {
+    shape_of<cfg_big>(), shape_of<cfg_glu>(),   shape_of<cfg_o>(),       shape_of<cfg_small>(), shape_of<cfg_mid>(),
+    shape_of<cfg_mid2>(), shape_of<cfg_tiny2>(), shape_of<cfg_tiny2x2>(), shape_of<cfg_tiny>(),
+};
+
+// The launch cost model, in microseconds. U = T * S units (T tiles in S K
+// splits) on P CUs. A unit runs its K-steps (nk / (S * kg)) and `prologue` more
+// (the pipeline's fill and the epilogue); a step takes `step` in a workgroup
+// that has a nearly idle GPU for itself, and busy() times that in all the rounds
+// of a launch: the clock falls under the power limit and the L2s fill up with
+// the share of CUs at work, and workgroups that share a CU slow each other. A
+// split launch pays for its partial sums: each unit writes its tile and the
+// last ones read them back, 2 * U * BM*BN*4 bytes at 8 TB/s over `partial`, and
+// `split` a split for their round trips. Where the weights and the output
+// outgrow the 256 MB last-level cache, a launch takes up to 1 + `cold` times as
+// long (from 200 to 400 MB). Each kind of launch has rates of its own: the
+// epilogues cost differently, and a group's activations come from a norm where
+// one weight's come from the packer, which stores past the caches. The mixed
+// launch has too: its half tiles have another layout of waves than the 128x128
+// tiles alone.
+//
+// The numbers are fits to 17000 launches timed plan after plan, each behind
+// the kernel that makes its activations (a norm, a GLU or the packer), as the
+// first reads of an operand that no L2 holds yet are a good part of a short
+// launch: least squares, then a descent on the choice itself, after which two
+// rates were moved by hand to where the choice lost least (128x128 tiles of one
+// weight up by 5%, 256x128 tiles of 4 waves in a group down by 7%). The launches
+// span single weights of any width, q/k/v and gate/up groups, heads of up to
+// 151936 columns, residual and fused launches, 32 to 4096 rows, K 256 to 17408.
+// Over them the choice takes 0.2 (fused) to 1.1% (one weight) longer than the
+// fastest plan measured, the worst hundredth 3 to 13%.
+enum launch_class { CLASS_SINGLE, CLASS_RESIDUAL, CLASS_GROUP, CLASS_FUSED, CLASSES };
+
+struct launch_rate {
+    double fixed, prologue, step;
+    double load[6];  // busy()
+    double split, partial, cold;
+};
+
+// {}: a shape that the kind does not take
+constexpr launch_rate RATES[CLASSES][SHAPES] = {
+    {   // one weight
+     {},
+     {2.0349, 6.6824, 0.5278, {0.2952}, 2.4903, 0.5995, 0.1122},
+     {1.7754, 14.2972, 0.3707, {0.4091}, 2.1513, 0.169, 0.0222},
+     {1.9307, 3.4291, 0.4488, {0.1525}, 1.3371, 1.0892, 0.1335},
+     {0, 3.0762, 0.3477, {0.1863, 1.4931, 1.3741}, 1.1467, 1.0997, 0.3409},
+     {0.4572, 2.3648, 0.4867, {0.0891}, 1.1198, 1.8362, 0.2082},
+     {1.3166, 1.1414, 0.349, {0.158}, 0.8535, 1.2643, 0.4217},
+     {0.899, 2.84, 0.4333, {0.2195, 1.5544, 1.5184}, 0.7542, 0.6682, 0.4942},
+     {0, 4.5243, 0.3027, {0.1582, 1.3153, 1.6153, 2.1583, 0.5474, 0.1096}, 0.8015, 0.7724, 0.6799},
+    },
+    {   // one weight, residual
+     {4.6875, 13.8007, 0.4665, {0.659}, 0.861, 0.4655, 0},
+     {4.7149, 9.1415, 0.461, {0.7206}, 0.7762, 0.4472, 0.0057},
+     {1.6817, 15.8825, 0.3601, {0.4075}, 1.8692, 0.1466, 0.032},
+     {2.5852, 13.9579, 0.3095, {0.5498}, 1.1535, 0.2057, 0.0697},
+     {0.9722, 9.8312, 0.2547, {0.4533, 1.707, 1.9024}, 0.8829, 0.3954, 0.2392},
+     {1.5205, 7.0075, 0.3579, {0.3598}, 0.7499, 1.7591, 0.0743},
+     {2.0204, 4.8614, 0.2738, {0.2693}, 0.5265, 1.3108, 0.1},
+     {1.6391, 4.7094, 0.3661, {0.3302, 1.6946, 1.6861}, 0.5636, 0.7032, 1.0184},
+     {1.8307, 6.2391, 0.2095, {0.3796, 1.8189, 2.1157, 2.7646, 0.7054, 0.1742}, 0.5884, 0.4164, 0.6617},
+    },
+    {   // a group
+     {4.632, 7.3286, 0.4373, {0.4991}, 3.0005, 0.1132, 0.0692},
+     {3.4579, 7.0427, 0.4462, {0.5159}, 1.8586, 0.3202, 0.048},
+     {2.0923, 7.5832, 0.3804, {0.3522}, 2.1902, 0.4381, 0.0116},
+     {2.0139, 6.3952, 0.3075, {0.4969}, 1.7265, 0.4282, 0.058},
+     {1.6618, 4.9488, 0.259, {0.2956, 1.6625, 1.841}, 1.0306, 0.8483, 0.0275},
+     {1.964, 3.1205, 0.4234, {0.2743}, 0.8497, 0.9997, 0},
+     {2.992, 1.814, 0.2916, {0.3084}, 0.8149, 0.0729, 0},
+     {3.0795, 1.6498, 0.3942, {0.123, 1.6706, 1.6649}, 0.5748, 1.4268, 0},
+     {1.9724, 3.8809, 0.2715, {0.1591, 1.4708, 1.6243, 2.234, 0.6013, 0.222}, 0.8035, 0.601, 0},
+    },
+    {   // fused GLU
+     {},
+     {2.1605, 8.4353, 0.4916, {0.3945}, 0.5585, 0.6701, 0.0555},
+     {},
+     {0.8151, 7.7693, 0.3619, {0.2423}, 1.8657, 0.4195, 0.0294},
+     {2.1204, 4.8003, 0.2559, {0.1894, 1.8192, 1.8119}, 0, 1.5729, 0.0718},
+     {1.9759, 3.2529, 0.4401, {0.1593}, 0.3617, 1.9569, 0},
+     {2.266, 1.902, 0.3876, {0}, 0.805, 1.1022, 0},
+     {1.326, 3.7091, 0.4531, {0.1083, 1.6447, 1.3917}, 0.2779, 2.9564, 0},
+     {1.8356, 5.4968, 0.2744, {0.0615, 1.5575, 1.8098, 2.356, 0.5662, 0.1817}, 0, 1.6553, 0},
+    },
+};
+
+// `whole`: a step in a whole round of 256x128 tiles; `half`, `half_prologue`
+// and `half_load` as step, prologue and load[0] for the half tiles
+struct mixed_rate {
+    double fixed, prologue, whole, half, half_prologue, half_load, cold;
+};
+
+constexpr mixed_rate MIXED_RATES[CLASS_FUSED] = {
+    {0, 13.1187, 0.5858, 0.5442, 0, 0.2438, 0.1086},
+    {0, 14.8117, 0.7393, 0.3424, 18.3353, 0.6001, 0},
+    {4.063, 6.9994, 0.6551, 0.3497, 5.0218, 0.3923, 0.0503},
+};
+
+// A step's time over a lone workgroup's, summed over the rounds of `units`
+// units on P CUs. One workgroup a CU: whole rounds and a last, partly filled
+// one, a round rising to 1 + load[0] with the square of the share of CUs. Two:
+// to 1 + load[0] with one on each CU, then, once any CU has two, on a line from
+// load[1] to load[2]. Up to five: a staircase by the CU with the most, 1 +
+// load[0], load[1], load[2], load[3], then load[4] times their number, its
+// steps sloped by load[5].
+double busy(int per_cu, const double * load, double units, double P) {
+    const double q = units / P;
+    if (per_cu == 1) {
+        const double n = std::floor(q), f = q - n;
+        return n * (1 + load[0]) + (f > 0 ? 1 + load[0] * f * f : 0.0);
+    }
+    if (per_cu == 2) {
+        const double n = std::floor(q / 2), f = q / 2 - n;
+        if (f == 0) return n * load[2];
+        return n * load[2] + (f <= 0.5 ? 1 + load[0] * 4 * f * f : load[1] + (load[2] - load[1]) * (2 * f - 1));
+    }
+    const double c = std::ceil(q);
+    if (c <= 1) return 1 + load[0] * q * q;
+    return (c <= 4 ? load[(int) c - 1] : load[4] * c) + load[5] * (q - (c - 1));
+}
+
+// What a plan is made from: a launch's sizes on P CUs.
+struct launch_sizes {
+    int64_t M;
+    int nk, nw;
+    int64_t N[ZEST_GEMM_MAX_GROUP];
+    int64_t P;
+
+    // tiles of one shape
+    int64_t tiles(int bm, int bn) const {
+        int64_t nt = 0;
+        for (int i = 0; i < nw; i++) nt += (N[i] + bn - 1) / bn;
+        return (M + bm - 1) / bm * nt;
+    }
+
+    // 0 with everything in the last-level cache, 1 with nothing
+    double cold(int cls) const {
+        double n = 0, k = (double) nk * ZEST_TILE_K;
+        for (int i = 0; i < nw; i++) n += (double) N[i];
+        const double out = cls == CLASS_RESIDUAL ? 8.0 : cls == CLASS_FUSED ? 1.0 : 4.0;  // bytes a column
+        const double mb = (n * k * 1.125 + (double) M * (n * out + k * 2)) / 1e6;
+        return std::min(1.0, std::max(0.0, (mb - 200) / 200));
+    }
+};
+
+launch_sizes sizes_of(const gemm_params & p, const int64_t * N, int64_t P) {
+    launch_sizes z{p.M, p.nk, p.nw, {}, P};
+    for (int i = 0; i < p.nw; i++) z.N[i] = N[i];
+    return z;
+}
+
+// What splitting K costs: grows with S.
+double split_us(int cls, int k, int64_t T, int S) {
+    if (S == 1) return 0.0;
+    const launch_rate & r = RATES[cls][k];
+    return r.split * S + r.partial * 2.0 * (double) (T * S) * TILES[k].bm * TILES[k].bn * 4 / 8e6;
+}
+
+double plan_us(int cls, int k, int64_t T, int S, const launch_sizes & z, double cold) {
+    const launch_rate & r = RATES[cls][k];
+    const tile_shape & t = TILES[k];
+    const double steps = (double) z.nk / (S * t.kg) + r.prologue;
+    const double us = r.fixed + steps * r.step * busy(t.per_cu, r.load, (double) (T * S), (double) z.P);
+    return (us + split_us(cls, k, T, S)) * (1 + r.cold * cold);
+}
+
 // A launch's plan: its tile shape, K splits and, for a mixed launch, how many
 // of its 256x128 tiles run whole.
 struct gemm_plan {
@@ -1475,44 +1599,61 @@ struct gemm_plan {
     int splits = 1;
     int64_t nbig = 0;
     double us = 1e300;
+
+    const tile_shape & tile() const { return TILES[kind == SHAPE_MIXED ? (int) SHAPE_GLU : kind]; }
 };
 
 // The split-K workspace of T tiles of shape k in S splits.
-size_t partial_bytes_of(int k, int64_t T, int S) { return (size_t) (T * S) * RATES[k].bm * RATES[k].bn * 4; }
-size_t counters_of(int k, int64_t T) { return (size_t) T * RATES[k].waves; }
+size_t partial_bytes_of(int k, int64_t T, int S) { return (size_t) (T * S) * TILES[k].bm * TILES[k].bn * 4; }
+size_t counters_of(int k, int64_t T) { return (size_t) T * TILES[k].waves; }
 
-// The cheapest plan of a plain (or residual) launch by the cost model: a tile
-// shape with its K splits, or a mixed launch. A launch whose whole tiles fill
-// every CU is not split, a split
-// keeps at least three K-steps a K-group, and the partial sums of K up to 32768
-// fit the static workspace of zest_gemm_group_noalloc, which runs the same
-// plan (only a longer K is worth more: 2048 x 2816 x 65536 in four splits).
-gemm_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P, int max_splits) {
-    gemm_plan best;
-    bool whole = true;  // every weight whole 160-row tiles
-    for (int i = 0; i < p.nw; i++) whole &= N[i] % cfg_o::BN == 0;
+// 128x160 tiles need weights of whole 160-row tiles
+bool whole_o_tiles(const launch_sizes & z) {
+    bool whole = true;
+    for (int i = 0; i < z.nw; i++) whole &= z.N[i] % cfg_o::BN == 0;
+    return whole;
+}
+
+// The mixed launch's plan: whole rounds of 256x128 tiles, the part-round left
+// as half tiles. Its us stays 1e300 where there is none.
+gemm_plan plan_mixed(int cls, const launch_sizes & z) {
+    const int64_t T = z.tiles(cfg_glu::BM, cfg_glu::BN), R = T / z.P, rem = T % z.P;
+    gemm_plan plan;
+    if (R < 1 || rem == 0 || R * z.P % 8 != 0) return plan;
+    const mixed_rate & m = MIXED_RATES[cls];
+    const double whole = (double) R * (z.nk + m.prologue) * m.whole;
+    const double half = (z.nk + m.half_prologue) * m.half * busy(1, &m.half_load, 2.0 * rem, (double) z.P);
+    return {SHAPE_MIXED, 1, R * z.P, (m.fixed + whole + half) * (1 + m.cold * z.cold(cls))};
+}
+
+// The cheapest plan of a plain launch by the cost model: a tile shape with its
+// K splits, or a mixed launch. A launch whose whole tiles give every CU one (two
+// of the one-group 64x64 tiles) is not split: the largest gain of it measured
+// there is 1%. A split keeps at least three K-steps a K-group, and the partial
+// sums of K up to 32768 fit the static workspace of zest_gemm_group_noalloc,
+// which runs the same plan (only a longer K is worth more: 2048 x 2816 x 65536
+// in four splits).
+gemm_plan plan_plain(const launch_sizes & z, int max_splits) {
+    const int cls = z.nw > 1 ? CLASS_GROUP : CLASS_SINGLE;
+    gemm_plan best = plan_mixed(cls, z);
+    const bool whole = whole_o_tiles(z);
+    const double cold = z.cold(cls);
     for (int k = 0; k < SHAPES; k++) {
-        const shape_rate & r = RATES[k];
-        if (k == SHAPE_O && !whole) continue;
-        const int64_t T = tiles_of(p, N, r.bm, r.bn), slots = P * r.per_cu;
+        const tile_shape & t = TILES[k];
+        const launch_rate & r = RATES[cls][k];
+        if (r.step == 0 || (k == SHAPE_O && !whole)) continue;
+        const int64_t T = z.tiles(t.bm, t.bn), most = z.P * (t.per_cu > 2 ? 2 : 1);
         for (int S = 1; S <= max_splits; S++) {
-            if (S > 1 && (T >= slots || T * S > 4 * slots || p.nk < 3 * S * r.kg)) break;
-            if (S > 1 && (p.nk <= 512 || whole) &&
+            if (S > 1 && (T >= most || T * S > 4 * z.P * std::min(t.per_cu, 2) || z.nk < 3 * S * t.kg)) break;
+            if (S > 1 && (z.nk <= 512 || whole) &&
                 (partial_bytes_of(k, T, S) > ZEST_NOALLOC_PARTIAL_BYTES || counters_of(k, T) > ZEST_NOALLOC_COUNTERS))
                 break;
-            if (r.kg > 1 && (p.nk % (S * r.kg) || p.nk < 2 * S * r.kg)) continue;
-            const double us = plan_us(r, T, p.nk, P, S);
+            // no more splits can win (the rest of this one's time is at least that of its first steps)
+            if (S > 1 && r.fixed + r.prologue * r.step + split_us(cls, k, T, S) >= best.us) break;
+            if (t.kg > 1 && (z.nk % (S * t.kg) || z.nk < 2 * S * t.kg)) continue;
+            const double us = plan_us(cls, k, T, S, z, cold);
             if (us < best.us) best = {k, S, 0, us};
         }
-    }
-    // whole rounds of 256x128 tiles, the part-round left as half tiles (its
-    // launch has no gap between the two: measured 4% under the sum)
-    const int64_t T = tiles_of(p, N, cfg_glu::BM, cfg_glu::BN), R = T / P, rem = T % P;
-    if (R >= 1 && rem > 0 && R * P % 8 == 0) {
-        const shape_rate & w = RATES[SHAPE_GLU];
-        const double us =
-            0.96 * (w.fixed + rounds_us(w, R * P, p.nk, P) + rounds_us(RATES[SHAPE_SMALL], 2 * rem, p.nk, P));
-        if (us < best.us) best = {SHAPE_MIXED, 1, R * P, us};
     }
     return best;
 }
@@ -1523,24 +1664,33 @@ gemm_plan plan_plain(const gemm_params & p, const int64_t * N, int64_t P, int ma
 // zeros (with 64-column tiles and F % 64 == 32 the last tile would end at F).
 int64_t glu_columns(int64_t N) { return (N + 127) / 128 * 128; }
 
-// The plan of a launch with epilogue `epi`. A fused GLU launch splits K as the
-// plain launch of its 2F columns would, in as many K-groups (so its gate and
-// up sums are that launch's, bit for bit: a sum depends on the K-steps'
-// partition and order, not on the tile shape), and takes the cheapest of its
-// tile shapes for that partition.
-gemm_plan plan_of(int epi, const gemm_params & p, const int64_t * N, int64_t P, int max_splits) {
-    const gemm_plan plain = plan_plain(p, N, P, max_splits);
-    if (epi < 0) return plain;
-    const int64_t Nt = glu_columns(N[0]);
-    const int kg = plain.kind == SHAPE_MIXED ? 1 : RATES[plain.kind].kg;
+// The plan of a launch with epilogue `epi`. A residual launch and a fused GLU
+// launch split K as the plain launch of their columns would, in as many
+// K-groups (so their sums are that launch's, bit for bit: a sum depends on the
+// K-steps' partition and order, not on the tile shape), and take the cheapest
+// of their tile shapes for that partition.
+gemm_plan plan_of(int epi, const launch_sizes & z, int max_splits) {
+    const gemm_plan plain = plan_plain(z, max_splits);
+    if (epi == EPI_PLAIN) return plain;
+    const int cls = epi == EPI_RESIDUAL ? CLASS_RESIDUAL : CLASS_FUSED, S = plain.splits;
+    const double cold = z.cold(cls);
     gemm_plan best;
-    for (const int k : {SHAPE_GLU, SHAPE_SMALL, SHAPE_MID, SHAPE_MID2, SHAPE_TINY2, SHAPE_TINY2X2}) {
-        const shape_rate & r = RATES[k];
-        if (r.kg != kg) continue;
-        const double us = plan_us(r, tiles_of(p, &Nt, r.bm, r.bn), p.nk, P, plain.splits);
-        if (us < best.us) best = {k, plain.splits, 0, us};
+    launch_sizes y = z;
+    if (cls == CLASS_FUSED) y.N[0] = glu_columns(z.N[0]);
+    else if (S == 1 && plain.tile().kg == 1) best = plan_mixed(cls, z);
+    for (int k = 0; k < SHAPES; k++) {
+        const tile_shape & t = TILES[k];
+        if (RATES[cls][k].step == 0 || t.kg != plain.tile().kg || (k == SHAPE_O && !whole_o_tiles(z))) continue;
+        const double us = plan_us(cls, k, y.tiles(t.bm, t.bn), S, y, cold);
+        if (us < best.us) best = {k, S, 0, us};
     }
     return best;
+}
+
+// The tiles of a plan.
+int64_t plan_tiles(int epi, const gemm_plan & plan, launch_sizes z) {
+    if (epi >= 0) z.N[0] = glu_columns(z.N[0]);
+    return z.tiles(plan.tile().bm, plan.tile().bn);
 }
 
 // Plans and launches a GEMM. A split-K plan takes its workspace from `fixed`
@@ -1553,13 +1703,14 @@ int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const ch
                const sk_space * fixed = nullptr) {
     int dev = 0;
     (void) hipGetDevice(&dev);
-    const int64_t P = cu_count(dev), Nt = glu_columns(N[0]);
+    const int64_t Nt = glu_columns(N[0]);
     const int64_t * cols = EPI >= 0 ? &Nt : N;
-    gemm_plan pp = plan_of(EPI, p, N, P, ZEST_GEMM_MAX_SPLIT);
+    const launch_sizes z = sizes_of(p, N, cu_count(dev));
+    gemm_plan pp = plan_of(EPI, z, ZEST_GEMM_MAX_SPLIT);
     std::unique_lock<std::mutex> lock(g_sk_mu, std::defer_lock);
     sk_space sp;
     if (pp.splits > 1) {
-        const int64_t T = tiles_of(p, cols, RATES[pp.kind].bm, RATES[pp.kind].bn);
+        const int64_t T = plan_tiles(EPI, pp, z);
         const size_t partial_bytes = partial_bytes_of(pp.kind, T, pp.splits), n_counters = counters_of(pp.kind, T);
         if (fixed) {
             if (partial_bytes > fixed->partial_bytes || n_counters > fixed->n_counters)
@@ -1574,7 +1725,7 @@ int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const ch
             lock.lock();
             const int st = sk_reserve(s, partial_bytes, n_counters, sp, name);
             if (st != ZEST_OK) return st;
-            if (!sp.partial) pp = plan_of(EPI, p, N, P, 1);
+            if (!sp.partial) pp = plan_of(EPI, z, 1);
         }
     }
     const int S = pp.splits;
@@ -1585,6 +1736,7 @@ int launch_any(const gemm_params & p, const int64_t * N, hipStream_t s, const ch
         case SHAPE_MID2: return launch<cfg_mid2, EPI>(p, cols, S, sp, s, name);
         case SHAPE_TINY2: return launch<cfg_tiny2, EPI>(p, cols, S, sp, s, name);
         case SHAPE_TINY2X2: return launch<cfg_tiny2x2, EPI>(p, cols, S, sp, s, name);
+        case SHAPE_TINY: return launch<cfg_tiny, EPI>(p, cols, S, sp, s, name);
         default: break;
     }
     if constexpr (EPI < 0) {
@@ -1723,11 +1875,11 @@ extern "C" int zest_gemm_plan(int kind, int64_t M, int64_t K, int n, const int64
     static_assert(ZEST_PLAN_PLAIN == EPI_PLAIN && ZEST_PLAN_RESIDUAL == EPI_RESIDUAL, "a plan's kinds are the epilogues");
     gemm_params p = base_params(nullptr, M, K, nullptr);
     p.nw = n;
-    const gemm_plan plan = plan_of(kind, p, N, cus, ZEST_GEMM_MAX_SPLIT);
-    const bool mixed = plan.kind == SHAPE_MIXED;
-    const shape_rate & t = RATES[mixed ? (int) SHAPE_GLU : plan.kind];
-    const int64_t Nt = glu_columns(N[0]), T = tiles_of(p, kind >= 0 ? &Nt : N, t.bm, t.bn);
-    *out = {t.bm, t.bn, t.waves, t.kg, t.per_cu, plan.splits, T, mixed ? plan.nbig : T,
+    const launch_sizes z = sizes_of(p, N, cus);
+    const gemm_plan plan = plan_of(kind, z, ZEST_GEMM_MAX_SPLIT);
+    const tile_shape & t = plan.tile();
+    const int64_t T = plan_tiles(kind, plan, z);
+    *out = {t.bm, t.bn, t.waves, t.kg, t.per_cu, plan.splits, T, plan.kind == SHAPE_MIXED ? plan.nbig : T,
             plan.splits > 1 ? (int64_t) partial_bytes_of(plan.kind, T, plan.splits) : 0};
     return ZEST_OK;
 }

@@ -29,7 +29,7 @@ def k_steps(k):
     return (k + 63) // 64
 
 
-# (BM, BN, consumer waves) of cfg_big, cfg_small, cfg_glu and cfg_tiny
+# (BM, BN, consumer waves) of cfg_big, cfg_small, cfg_glu and cfg_tiny (64x64 tiles of one K-group)
 CONFIGS = [(256, 128, 4), (128, 128, 4), (256, 128, 8), (64, 64, 2)]
 
 
@@ -153,7 +153,7 @@ def test_scalar_offsets_stay_inside_operands(M, N, K):
     nk = k_steps(K)
     for (BM, BN, CWM), S in itertools.product(CONFIGS, range(1, 17)):
         if S > 1 and nk // S < 4:
-            continue  # the planner never splits below four steps a split
+            continue  # shorter splits: test_small_tile_shapes_stay_inside_operands
         check_launch(M, N, K, BM, BN, CWM, S)
     # 64x64 tiles as two K-groups (cfg_tiny2), in every split count the
     # launch accepts (nk a multiple of splits x groups)
@@ -169,10 +169,14 @@ def test_scalar_offsets_stay_inside_operands(M, N, K):
 def test_small_tile_shapes_stay_inside_operands(M, N, K):
     # cfg_mid, and cfg_mid2, cfg_tiny2 and cfg_tiny2x2 as two K-groups, in
     # every split the planner can give them (three steps a K-group at least);
-    # cfg_small's rows (4 row blocks, two column blocks); cfg_o in K splits
+    # cfg_small's rows (4 row blocks, two column blocks); cfg_o in K splits;
+    # cfg_tiny and both 256x128 shapes
     nk = k_steps(K)
     for S in range(1, 17):
         if S == 1 or nk >= 3 * S:
+            check_launch(M, N, K, 64, 64, 2, S)
+            check_launch(M, N, K, 256, 128, 4, S)
+            check_launch(M, N, K, 256, 128, 8, S)
             check_launch(M, N, K, 128, 64, 4, S)
             check_launch(M, N, K, 128, 128, 4, S)
             if N % 160 == 0:
@@ -184,7 +188,7 @@ def test_small_tile_shapes_stay_inside_operands(M, N, K):
 
 # (BM, BN, consumer waves across rows, across columns, K-groups, workgroups a CU)
 LDS_SHAPES = [(256, 128, 4, 1, 1, 1), (256, 128, 8, 1, 1, 1), (128, 160, 4, 1, 1, 1), (128, 128, 4, 2, 1, 1),
-              (128, 64, 4, 1, 1, 2), (128, 64, 4, 1, 2, 1), (64, 64, 2, 1, 2, 1), (64, 64, 2, 1, 2, 2)]
+              (128, 64, 4, 1, 1, 2), (128, 64, 4, 1, 2, 1), (64, 64, 2, 1, 2, 1), (64, 64, 2, 1, 2, 2), (64, 64, 2, 1, 1, 5)]
 
 
 @pytest.mark.parametrize("BM,BN,CWM,CWN,KG,MINB", LDS_SHAPES)

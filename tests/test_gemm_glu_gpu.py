@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+from gemm_plans import FUSED, plan_name
 from gen import Rng, wide_blocks
 from helpers import load_quant, nrmse
 
@@ -70,9 +71,9 @@ def separate(z, kind, a, m, gate, up, wtype, f, k):
     (8, 1024, 2560, 1536),
     (12, 520, 8960 // 10, 1536),
     (12, 2048, 9728, 2560),  # BASELINE config 2's gate/up: 2048 x 9728 x 2560, Q4_K
-    (8, 2048, 1024, 9728),   # few tiles, long K: the launch splits K
-    (0, 2048, 3072, 512),    # 384 tiles: a round and a half, the half as 128-row tiles
-    (0, 1500, 4096, 512),    # 6 x 64 = 384 tiles, ragged rows: persistent workgroups
+    (8, 2048, 1024, 9728),   # few tiles, long K
+    (0, 2048, 3072, 512),    # 384 tiles of 256x128: a round and a half
+    (0, 1500, 4096, 512),    # ragged rows, three rounds of 128x64 tiles
 ])
 def test_gemm_glu_matches_unfused_swiglu(zest_gpu, oracle, wtype, M, F, K):
     import torch
@@ -138,8 +139,8 @@ def test_order_sensitive_operands_show_another_k_split(zest_gpu):
 @pytest.mark.parametrize("M,F,K", [
     (520, 896, 1536),   # 252 tiles of 64x64, each K-split between two K-groups
     (1024, 512, 4096),  # 256 of them, K 4096
-    (2048, 1024, 8192),  # few tiles, long K: split
-    (256, 512, 4096),    # 64 tiles of 64x64 in two K-groups and four K splits
+    (2048, 1024, 8192),  # few tiles, long K
+    (256, 512, 4096),    # 64 tiles of 64x64 in two K-groups and K splits
     (2048, 6144, 4096),  # three rounds: persistent workgroups
     (1500, 4096, 4096),
 ])
@@ -157,20 +158,16 @@ def test_gemm_glu_bit_exact_order_sensitive(zest_gpu, M, F, K):
     assert torch.equal(xo, x_ref), (M, F, K)
 
 
-@pytest.mark.parametrize("M,F,K", [
-    (300, 1664, 1536),   # 128x64 tiles in two K-groups
-    (300, 2720, 1280),   # the plain launch so, the fused one as 64x64 tiles, two workgroups a CU
-    (600, 800, 1280),    # the plain launch as 64x64 tiles, the fused one as 128x64, both two K-groups
-    (129, 96, 2560),     # 64x64 tiles in two K-groups and two K splits
-    (129, 32, 3072),     # and three
-    (129, 2592, 64),     # 128x64 tiles of one K-step
-    (600, 1024, 3080),   # an odd number of K-steps: no K-groups
-    (1000, 1760, 1280),  # the plain launch as 128x64 tiles, the fused one as 128x128
-    (600, 2880, 1536),   # 128x128 tiles, 16 waves
-    (600, 3520, 1536),   # the plain launch as 128x160 tiles, the fused one as 256x128
+@pytest.mark.parametrize("M,F,K,shape,splits", FUSED + [
+    (129, 2592, 64, None, 1),      # one K-step
+    (600, 1024, 3080, None, 1),    # an odd number of K-steps: no K-groups
 ])
-def test_gemm_glu_planned_shapes(zest_gpu, M, F, K):
-    """The fused launch's tile shapes give the plain launch's sums whatever shape that one takes."""
+def test_gemm_glu_planned_shapes(zest_gpu, M, F, K, shape, splits):
+    """The fused launch's tile shapes, split and unsplit, give the plain launch's sums whatever shape that one takes,
+    and write the operand's padding."""
+    import torch
+    if shape and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert plan_name(zest_gpu, M, [2 * F], K, 2) == (shape, splits)
     test_gemm_glu_bit_exact_order_sensitive(zest_gpu, M, F, K)
     test_gemm_glu_writes_the_operand_padding(zest_gpu, M, F, K)
 
@@ -197,7 +194,7 @@ def test_gemm_glu_writes_the_operand_padding(zest_gpu, M, F, K):
 
 @pytest.mark.parametrize("M,F,K", [
     (300, 160, 256),    # 6 tiles: one workgroup a tile
-    (1500, 4096, 512),  # 384 tiles: persistent workgroups, each kind's own kernel
+    (1500, 4096, 1536),  # 384 tiles of 256x128: persistent workgroups, each kind's own kernel
 ])
 @pytest.mark.parametrize("kind", list(KINDS))
 def test_gemm_glu_every_kind(zest_gpu, kind, M, F, K):

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+from gemm_plans import PLAIN, RESIDUAL, plan_name
 from gen import Rng, make_data, wide_blocks
 from helpers import gemm_check, load_quant
 
@@ -17,6 +18,11 @@ pytestmark = pytest.mark.gpu
 def _dev(a):
     import torch
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _cus():
+    import torch
+    return torch.cuda.get_device_properties(0).multi_processor_count
 
 
 def run_gemm(z, x: np.ndarray, wtype: int, raw: np.ndarray, n: int):
@@ -102,7 +108,7 @@ def test_general_blocks_among_zero_blocks(zest_gpu, oracle, M, N, K):
     (8, 1, 256, 512),
     (12, 2048, 1024, 2560),  # K/V projection of config 3
     (8, 1024, 1024, 4096),   # 64x64 tiles, one a CU, each in two K-groups
-    (8, 256, 1024, 4096),    # 64 of them, in two K-groups and four K splits
+    (8, 256, 1024, 4096),    # 64 of them, in two K-groups and K splits
 ])
 def test_gemm_against_oracle(zest_gpu, oracle, wtype, M, N, K):
     import torch
@@ -126,27 +132,15 @@ def test_gemm_against_oracle(zest_gpu, oracle, wtype, M, N, K):
     assert maxrel32 <= 1e-3
 
 
-@pytest.mark.parametrize("M,ns,K", [
-    (777, [2050], 1000),            # 128x64 tiles in two K-groups; ragged rows, columns and K
-    (200, [2050], 5120),            # and in two K splits
-    (129, [64], 64),                # one K-step, 128x64 tiles
-    (1000, [1119], 3208),           # 128x64 tiles, two a CU, an odd number of K-steps
-    (511, [1600], 4104),            # in three K splits
-    (129, [200], 4104),             # in four: two rounds of the fixup
-    (1300, [2400], 3072),           # 128x128 tiles, 16 waves
-    (100, [1000], 2560),            # 64x64 tiles in two K-groups and two K splits
-    (777, [96], 3072),              # and three
-    (33, [200], 5120),              # and four
-    (48, [9728, 9728], 2560),       # 304 of them, two workgroups a CU
-    (511, [3000], 5120),            # 128x64 tiles in two K-groups, 188 of them
-    (1300, [3000], 1280),           # 256x128 tiles, 8 consumers
-    (300, [800, 160, 35], 1024),    # a group
-    (768, [2560], 17408),           # 256x128 tiles in four K splits
+@pytest.mark.parametrize("M,ns,K,shape,splits", PLAIN + [
+    (129, [64], 64, "128x64", 1),   # one K-step
 ])
-def test_gemm_planned_shapes(zest_gpu, oracle, M, ns, K):
+def test_gemm_planned_shapes(zest_gpu, oracle, M, ns, K, shape, splits):
     """Every tile shape of the planner at ragged edges, with the K splits and K-groups it gives them, against fp64
     on the first, last and sampled rows (the bound of two roundings a product term of gemm_check); the residual
     form is the plain one plus the add, bit for bit; nothing outside the output's columns is written."""
+    if len(ns) * K > 64 and _cus() == 256:
+        assert plan_name(zest_gpu, M, ns, K) == (shape, splits)
     import torch
     x = Rng(M + sum(ns)).normal(M * K).reshape(M, K)
     a = zest_gpu.pack_act_x(torch.from_numpy(x).cuda())
@@ -175,6 +169,33 @@ def test_gemm_planned_shapes(zest_gpu, oracle, M, ns, K):
         got = zest_gpu.gemm_residual(a, M, ws[0], n, K, res)
         torch.cuda.synchronize()
         assert torch.equal(got, outs[0][:, :n] + res)
+
+
+@pytest.mark.parametrize("M,ns,K,shape,splits", RESIDUAL)
+def test_gemm_residual_planned_shapes(zest_gpu, oracle, M, ns, K, shape, splits):
+    """Every tile shape that a residual launch takes (for the plain launch's K splits and K-groups): the bits of the
+    plain launch plus the add, on operands where a change of summation order shows, in place as well, the rows past M
+    of the residual holding NaN; and within the bound of fp64."""
+    import torch
+    z, N = zest_gpu, ns[0]
+    if _cus() == 256:
+        assert plan_name(z, M, ns, K, -2) == (shape, splits)
+    a = z.pack_act_x(_dev(wide_blocks(M, K, M + K)))
+    wp = z.convert_weight(0, _dev(wide_blocks(N, K, N + K, 0.02).view(np.uint8)), N, K)
+    h = torch.full((M + 64, N), float("nan"), device="cuda")
+    h[:M] = torch.from_numpy(Rng(M + N).normal(M * N).reshape(M, N)).cuda()
+    nf = torch.zeros(1, dtype=torch.int32, device="cuda")
+    plain = z.gemm(a, M, wp, N, K, nonfinite=nf)
+    want = z.add(plain, h[:M].contiguous())
+    out = z.gemm_residual(a, M, wp, N, K, h[:M], nonfinite=nf)
+    z.gemm_residual(a, M, wp, N, K, h[:M], out=h[:M], nonfinite=nf)
+    torch.cuda.synchronize()
+    assert int(nf.item()) == 0
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+    assert torch.equal(h[:M].view(torch.int32), want.view(torch.int32)) and bool(torch.isnan(h[M:]).all())
+    rows = np.unique(np.concatenate([[0, M - 1], np.linspace(0, M - 1, 12).astype(int)]))
+    r64, ab = oracle.mul_mat_f64(decoded(z, oracle, wp, N, K), decoded_act(z, oracle, a, M, K)[rows])
+    assert gemm_check(plain.cpu().numpy()[rows], r64, ab, K)[0] <= 1.0
 
 
 def test_gemm_full_size_ffn_properties(zest_gpu, oracle):
@@ -287,16 +308,18 @@ def test_gemm_group(zest_gpu, oracle, M, K, ns, wtype):
 
 @pytest.mark.parametrize("M,ns,K", [
     (2000, [2560], 4096),         # config 3's O projection with ragged rows: 256 tiles of 128 x 160
-    (1024, [5120], 1024),
+    (1024, [5120], 1024),         # whole 160-row tiles that 256x128 ones take
     (1500, [1600, 1760], 1024),   # a group of two weights, 252 tiles
     (2048, [2560], 9728),         # config 3's down projection: one unsplit round, not three K splits
 ])
 def test_gemm_160_row_tiles(zest_gpu, oracle, M, ns, K):
     # a launch that 256 x 128 tiles run in one round, unsplit, while 128 x 128
-    # tiles would take two, runs as 128 x 160 tiles when every weight is whole
+    # tiles would take two, may run as 128 x 160 tiles when every weight is whole
     # 160-row tiles: against the oracle; with the residual epilogue (rows past
     # M of the residual holding NaN), bit for bit the GEMM followed by the ADD
     import torch
+    if M != 1024 and _cus() == 256:
+        assert plan_name(zest_gpu, M, ns, K) == ("128x160", 1)
     x = Rng(M + 7).normal(M * K).reshape(M, K)
     a = zest_gpu.pack_act_x(_dev(x))
     ws = []
@@ -348,6 +371,9 @@ def test_gemm_rounds_equal_one_round_launches(zest_gpu, oracle, M, ns, K):
     alone = [zest_gpu.gemm(a, M, w, n, K) for w, n in zip(ws, ns)]
     torch.cuda.synchronize()
     assert int(nf.item()) == 0
+    if _cus() == 256:
+        assert plan_name(zest_gpu, M, ns, K) == (("mixed", 1) if sum(ns) == 5120 else ("256x128 of 8 waves", 1))
+        assert all(zest_gpu.gemm_plan(M, [n], K)["splits"] * zest_gpu.gemm_plan(M, [n], K)["k_groups"] == 1 for n in ns)
     for i in range(len(ns)):
         assert torch.equal(outs[i].view(torch.int32), alone[i].view(torch.int32)), i
     rows = np.unique(np.concatenate([np.linspace(0, M - 1, 32).astype(int), [255, 256, M - 1]]))
@@ -364,7 +390,10 @@ def test_gemm_part_round_as_half_tiles(zest_gpu, oracle):
     # the result equals, bit for bit, two launches over the column halves (192
     # whole tiles each), and the oracle within the GEMM bar. Order-sensitive
     # operands (blocks spread over 2^+-12).
-    M, N, K = 2048, 6144, 512
+    M, N, K = 2048, 6144, 1536
+    if _cus() == 256:
+        assert plan_name(zest_gpu, M, [N], K) == ("mixed", 1)
+        assert plan_name(zest_gpu, M, [N // 2], K) == ("256x128 of 8 waves", 1)
     x = wide_blocks(M, K, 3)
     w = wide_blocks(N, K, 4, 0.02)
     c, nf, a, wp = run_gemm(zest_gpu, x, 0, w.view(np.uint8), N)
@@ -395,11 +424,11 @@ def test_gemm_group_rejects_bad_counts(zest_gpu):
 @pytest.mark.parametrize("M,N,K", [
     (2048, 2560, 4096),   # config 3's O projection: h += O
     (2048, 2560, 9728),   # its down projection (one round of 128 x 160 tiles)
-    (300, 200, 256),      # ragged rows, 128x128 tiles
+    (300, 200, 256),      # ragged rows
     (1024, 1000, 512),    # a width that is not a tile multiple
-    (2048, 6144, 512),    # 384 tiles: a round and a half, the half as 128-row tiles
+    (2048, 6144, 512),    # 384 tiles of 256x128: a round and a half
     (1024, 1024, 4096),   # 64x64 tiles in two K-groups
-    (256, 1024, 4096),    # and in four K splits
+    (256, 1024, 4096),    # and in K splits
 ])
 def test_gemm_residual_is_gemm_then_add(zest_gpu, M, N, K):
     # the residual epilogue adds in the store: the same floats as the GEMM

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+from gemm_plans import FUSED, PLAIN, RESIDUAL, plan_name
 
 
 @pytest.mark.parametrize("kind", [-2, -1, 0, 2])
@@ -42,3 +43,34 @@ def test_plan_arguments(zest):
                 dict(m=1, ns=[8] * 5, k=8), dict(m=1, ns=[8, 8], k=8, kind=2), dict(m=1, ns=[8], k=8, kind=9)]:
         with pytest.raises(RuntimeError):
             zest.gemm_plan(**bad)
+
+
+@pytest.mark.parametrize("kind,cases", [(-1, PLAIN), (-2, RESIDUAL), (2, FUSED)])
+def test_labelled_cases_take_their_plans(zest, kind, cases):
+    for M, ns, K, shape, splits in cases:
+        ns = [2 * ns] if kind >= 0 else ns
+        assert plan_name(zest, M, ns, K, kind) == (shape, splits), (M, ns, K)
+
+
+def test_labelled_cases_cover_what_the_planner_takes(zest):
+    # every (shape, split or not) that each kind of launch takes over a wide sweep of sizes has a labelled case
+    rng = np.random.default_rng(3)
+    for kind, cases in ((-1, PLAIN), (-2, RESIDUAL), (2, FUSED)):
+        have = {(shape, splits > 1) for *_, shape, splits in cases}
+        seen = set()
+        for _ in range(6000):
+            M, K = int(np.exp(rng.uniform(np.log(32), np.log(4200)))), int(np.exp(rng.uniform(np.log(200), np.log(30000)))) // 8 * 8
+            ns = [max(1, int(np.exp(rng.uniform(np.log(64), np.log(20000)))) // 160) * 160]
+            if kind == -1 and rng.random() < 0.4:
+                ns.append(ns[0] // 480 * 160 + 160)
+            if kind >= 0:
+                ns = [max(1, ns[0] // 64) * 64]
+            shape, splits = plan_name(zest, M, ns, K, kind)
+            seen.add((shape, splits > 1))
+        assert seen <= have, (kind, seen - have)
+
+
+def test_mixed_launch_of_a_part_round(zest):
+    # q, k and v of the hidden-2560 layer at 2048 tokens: a round and a half of 256x128 tiles runs the half as halves
+    # (60.8 us, whole tiles 63.7, as timed when the two were last told apart)
+    assert plan_name(zest, 2048, [4096, 1024, 1024], 2560) == ("mixed", 1)
