@@ -1630,12 +1630,14 @@ gemm_plan plan_mixed(int cls, const launch_sizes & z) {
 // K splits, or a mixed launch. A launch whose whole tiles give every CU one (two
 // of the one-group 64x64 tiles) is not split: the largest gain of it measured
 // there is 1%. A split keeps at least three K-steps a K-group, and the partial
-// sums of K up to 32768 fit the static workspace of zest_gemm_group_noalloc,
-// which runs the same plan (only a longer K is worth more: 2048 x 2816 x 65536
-// in four splits).
+// sums fit the static workspace of zest_gemm_group_noalloc, which runs the same
+// plan. Only for K over 32768 may 256x128 tiles outgrow it, where that saves a
+// twentieth of the time (2048 x 2816 x 65536 in four splits): that entry point
+// refuses those. Weights of whole 160-row tiles stay inside it at any K, as it
+// has accepted them since they ran as one unsplit round of 128x160 tiles.
 gemm_plan plan_plain(const launch_sizes & z, int max_splits) {
     const int cls = z.nw > 1 ? CLASS_GROUP : CLASS_SINGLE;
-    gemm_plan best = plan_mixed(cls, z);
+    gemm_plan best = plan_mixed(cls, z), outgrown;
     const bool whole = whole_o_tiles(z);
     const double cold = z.cold(cls);
     for (int k = 0; k < SHAPES; k++) {
@@ -1645,17 +1647,18 @@ gemm_plan plan_plain(const launch_sizes & z, int max_splits) {
         const int64_t T = z.tiles(t.bm, t.bn), most = z.P * (t.per_cu > 2 ? 2 : 1);
         for (int S = 1; S <= max_splits; S++) {
             if (S > 1 && (T >= most || T * S > 4 * z.P * std::min(t.per_cu, 2) || z.nk < 3 * S * t.kg)) break;
-            if (S > 1 && (z.nk <= 512 || whole) &&
-                (partial_bytes_of(k, T, S) > ZEST_NOALLOC_PARTIAL_BYTES || counters_of(k, T) > ZEST_NOALLOC_COUNTERS))
-                break;
+            const bool fits = S == 1 || (partial_bytes_of(k, T, S) <= ZEST_NOALLOC_PARTIAL_BYTES &&
+                                         counters_of(k, T) <= ZEST_NOALLOC_COUNTERS);
+            if (!fits && (z.nk <= 512 || t.bm < 256 || whole)) break;
             // no more splits can win (the rest of this one's time is at least that of its first steps)
             if (S > 1 && r.fixed + r.prologue * r.step + split_us(cls, k, T, S) >= best.us) break;
             if (t.kg > 1 && (z.nk % (S * t.kg) || z.nk < 2 * S * t.kg)) continue;
             const double us = plan_us(cls, k, T, S, z, cold);
-            if (us < best.us) best = {k, S, 0, us};
+            gemm_plan & plan = fits ? best : outgrown;
+            if (us < plan.us) plan = {k, S, 0, us};
         }
     }
-    return best;
+    return outgrown.us * 1.05 < best.us ? outgrown : best;
 }
 
 // The columns that a fused GLU's tiles cover: the output operand's K padding

@@ -74,3 +74,21 @@ def test_mixed_launch_of_a_part_round(zest):
     # q, k and v of the hidden-2560 layer at 2048 tokens: a round and a half of 256x128 tiles runs the half as halves
     # (60.8 us, whole tiles 63.7, as timed when the two were last told apart)
     assert plan_name(zest, 2048, [4096, 1024, 1024], 2560) == ("mixed", 1)
+
+
+def test_no_alloc_workspace_bound(zest):
+    # plans fit the static array of zest_gemm_group_noalloc for every K up to 32768, and for weights of whole 160-row
+    # tiles at any K; others may outgrow it as 256x128 tiles, where the best plan that fits takes a twentieth longer
+    rng, most, over = np.random.default_rng(11), 64 << 20, 0
+    for _ in range(4000):
+        M = int(np.exp(rng.uniform(0, np.log(4200))))
+        K = int(np.exp(rng.uniform(np.log(1000), np.log(120000)))) // 8 * 8
+        N = int(np.exp(rng.uniform(np.log(64), np.log(17000)))) // 160 * 160 + (160 if rng.random() < 0.5 else 96)
+        p = zest.gemm_plan(M, [N], K)
+        if p["workspace"] > most:
+            over += 1
+            assert K > 32768 and p["tile_rows"] == 256 and N % 160, (M, N, K, p)
+    assert over < 100
+    assert zest.gemm_plan(2048, [2816], 65536)["workspace"] > most      # what the entry point refuses
+    for N in (2432, 2560, 2688):
+        assert zest.gemm_plan(2048, [N], 65536)["workspace"] <= most
