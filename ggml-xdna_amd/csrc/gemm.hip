@@ -1451,7 +1451,9 @@ constexpr tile_shape TILES[SHAPES] = {
 // first reads of an operand that no L2 holds yet are a good part of a short
 // launch: least squares, then a descent on the choice itself, after which two
 // rates were moved by hand to where the choice lost least (128x128 tiles of one
-// weight up by 5%, 256x128 tiles of 4 waves in a group down by 7%). The launches
+// weight up by 5%, 256x128 tiles of 4 waves in a group down by 7%) and the rates
+// of one weight's 256x128 tiles of 4 waves searched by themselves, the others
+// held (4096x8192x5120 takes them: 262.6 us, 267.7 as 8 waves). The launches
 // span single weights of any width, q/k/v and gate/up groups, heads of up to
 // 151936 columns, residual and fused launches, 32 to 4096 rows, K 256 to 17408.
 // Over them the choice takes 0.2 (fused) to 1.1% (one weight) longer than the
@@ -1467,7 +1469,7 @@ struct launch_rate {
 // {}: a shape that the kind does not take
 constexpr launch_rate RATES[CLASSES][SHAPES] = {
     {   // one weight
-     {},
+     {2.4286, 8.5589, 0.5328, {0.2485}, 2.3683, 0.6743, 0.0976},
      {2.0349, 6.6824, 0.5278, {0.2952}, 2.4903, 0.5995, 0.1122},
      {1.7754, 14.2972, 0.3707, {0.4091}, 2.1513, 0.169, 0.0222},
      {1.9307, 3.4291, 0.4488, {0.1525}, 1.3371, 1.0892, 0.1335},
