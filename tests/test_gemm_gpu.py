@@ -536,8 +536,9 @@ def test_gemm_random_shapes(zest_gpu, oracle):
 def test_gemm_random_shapes_order_sensitive(zest_gpu, oracle):
     # a wider seeded sweep on operands whose 8-value blocks span 2^+-12: rows
     # up to a few rounds of tiles (and across the 64-, 256- and 1024-row
-    # boundaries), widths up to 12288, K up to 4096, so the planner takes
-    # every tile shape, K split and K-group form; the plain, grouped and
+    # boundaries), widths up to 12288, K up to 4096: mostly unsplit plans of
+    # every tile width, K-groups among them (test_gemm_planned_shapes and its
+    # residual and fused twins hold the K splits); the plain, grouped and
     # residual launches against the oracle's bound, the residual added in
     # place bit-exact with the GEMM then ADD, and the fused GLU of every kind
     # bit-exact with the unfused chain, its operand written whole (padding
